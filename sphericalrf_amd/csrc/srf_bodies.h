@@ -47,6 +47,15 @@ constexpr uint32_t LOG_MAX_WORDS = 96;
 // consecutive addresses.  Runs without samples are not stored; the ray's word_mask says which are.
 struct StepLog { uint32_t* bits; float* t0; uint32_t stride; uint32_t words; };
 
+// What the writing march is made of: an entry per log word of a kept ray, in ray order and step order, so that consecutive entries'
+// samples lie one behind the other in the sample arrays.  A ray whose samples are not all in the log is one entry: it marches again.
+//   x  ray      y  log word | its rank among the ray's words << 8
+constexpr uint32_t ENTRY_MARCH = 0xffu;
+static_assert(LOG_MAX_WORDS < ENTRY_MARCH, "log words fit the entry");
+SRF_HD uint32_t train_ray_entries(const TrainRay& st) {
+	return st.logged ? (uint32_t)(__builtin_popcount(st.word_mask[0]) + __builtin_popcount(st.word_mask[1]) + __builtin_popcount(st.word_mask[2])) : 1u;
+}
+
 SRF_HD void step_log_flush(const StepLog& log, uint32_t i, uint32_t w, uint32_t word, float t_word, bool& logged, uint32_t* mask) {
 	if (!word || !logged) return;
 	if (w >= log.words) { logged = false; return; }
@@ -285,6 +294,7 @@ struct CountArgs {
 	Pcg32 rng;
 	TrainRay* state;
 	uint32_t* counts;
+	uint32_t* n_entries = nullptr;      // per ray: write entries it makes (train_ray_entries), or NULL
 	StepLog log;
 	SkipTable skip;
 	// parking: budget of probes per ray (0 = never park), the queue, its capacity, its fill counter; a wavefront only parks
@@ -317,6 +327,7 @@ SRF_HD void count_finish(CountLane& L, const CountArgs& A) {
 	st.word_mask[0] = L.mask[0]; st.word_mask[1] = L.mask[1]; st.word_mask[2] = L.mask[2];
 	A.state[L.i] = st;
 	A.counts[L.i] = L.j;
+	if (A.n_entries) A.n_entries[L.i] = train_ray_entries(st);
 	L.phase = LANE_IDLE;
 }
 
@@ -755,7 +766,6 @@ struct DirectSink {
 		if (sample_cell) sample_cell[k] = cell;
 	}
 };
-constexpr uint32_t WINDOW_EMPTY = 0xffffffffu;   // mark of a staging slot that no ray has written
 
 // occupancy_sampler.cu:644-688 — second march of a kept ray, writing its samples.  In pieces, so that a wavefront can
 // spread the per-sample work of its rays evenly over its lanes: the ray's own outputs, the replay of the step log
@@ -763,12 +773,10 @@ constexpr uint32_t WINDOW_EMPTY = 0xffffffffu;   // mark of a staging slot that 
 // grid up again for rays without a log.
 struct WriteRay { Vec3 o, d, wdir; uint32_t numsteps, base; float startt; };
 
-// occupancy_sampler.cu:644-664 — ray, target colour and sample range of kept ray i
-SRF_HD WriteRay train_write_ray(uint32_t i, const DatasetArgs& ds, const TrainRay& st, const uint32_t* counts, const uint32_t* base, const uint32_t* ray_index,
-                                float* rays_out, float* rays_rgba, uint32_t* numsteps_out) {
+// occupancy_sampler.cu:644-664 — ray, target colour and sample range of a kept ray, the r-th
+SRF_HD WriteRay train_write_ray(uint32_t r, const DatasetArgs& ds, const TrainRay& st, uint32_t count, uint32_t base, float* rays_out, float* rays_rgba, uint32_t* numsteps_out) {
 	WriteRay R;
-	R.numsteps = counts[i]; R.base = base[i]; R.startt = st.startt;
-	const uint32_t r = ray_index[i];
+	R.numsteps = count; R.base = base; R.startt = st.startt;
 	R.o = ld3(st.o); R.d = ld3(st.d);
 	st3(rays_out + 6 * (size_t)r, R.o);
 	st3(rays_out + 6 * (size_t)r + 3, R.d);
@@ -784,47 +792,21 @@ SRF_HD WriteRay train_write_ray(uint32_t i, const DatasetArgs& ds, const TrainRa
 	return R;
 }
 
-// the t chain inside the logged runs only; emit(j, t) for sample j of the ray, in order, until it returns false
+// the t chain from the first sample of a log word to its last; emit(j, t) for every sample, j counting on from the caller's
 template <class Emit>
-SRF_HD void train_write_replay(uint32_t i, const Params& P, const TrainRay& st, uint32_t cap, const StepLog& log, const Emit& emit) {
-	const float cone = P.cone_angle_constant;
-	const ShortForm f = disparity_short_form(P);
-	uint32_t j = 0;
-#if defined(__HIP_DEVICE_COMPILE__)
-	#pragma unroll
-#endif
-	for (uint32_t g = 0; g < 3; ++g) {      // unrolled: the mask words stay in registers
-		uint32_t m = st.word_mask[g];
-		// a word's bits and the t at its first sample are requested while the word before it is walked
-		uint32_t next_bits = 0u;
-		float next_t = 0.f;
-		if (m) {
-			const uint32_t w = g * 32u + (uint32_t)__builtin_ctz(m);
-			next_bits = log.bits[(size_t)w * log.stride + i];
-			next_t = log.t0[(size_t)w * log.stride + i];
+SRF_HD void train_replay_word(const Params& P, const ShortForm& f, uint32_t word, float t, uint32_t& j, uint32_t cap, const Emit& emit) {
+	if (!word) return;
+	word >>= (uint32_t)__builtin_ctz(word);
+	const bool short_form = f.usable && t >= f.t_lo;   // t only grows; the upper end is checked per step
+	ShortChain ch = short_chain_at(short_form ? t : 1.f);
+	while (word && j < cap) {
+		if (word & 1u) {
+			emit(j, t);
+			++j;
 		}
-		while (m) {
-			m &= m - 1u;
-			uint32_t word = next_bits;
-			float t = next_t;
-			if (m) {
-				const uint32_t w = g * 32u + (uint32_t)__builtin_ctz(m);
-				next_bits = log.bits[(size_t)w * log.stride + i];
-				next_t = log.t0[(size_t)w * log.stride + i];
-			}
-			word >>= (uint32_t)__builtin_ctz(word);
-			const bool short_form = f.usable && t >= f.t_lo;   // t only grows; the upper end is checked per step
-			ShortChain ch = short_chain_at(short_form ? t : 1.f);
-			while (word && j < cap) {
-				if (word & 1u) {
-					if (!emit(j, t)) return;
-					++j;
-				}
-				word >>= 1;
-				if (short_form && t <= f.t_hi) { ch = short_chain_next(f, ch); t = ch.t; }
-				else t += calc_dt(P, t, cone);      // beyond the short form's range for good: t only grows
-			}
-		}
+		word >>= 1;
+		if (short_form && t <= f.t_hi) { ch = short_chain_next(f, ch); t = ch.t; }
+		else t += calc_dt(P, t, P.cone_angle_constant);      // beyond the short form's range for good: t only grows
 	}
 }
 
@@ -883,13 +865,16 @@ SRF_HD void train_write_body(uint32_t i, const Params& P, const DatasetArgs& ds,
                              float* coords_out, const DirectSink& sink, StepLog log) {
 	if (!keep[i]) return;
 	const TrainRay st = state[i];
-	const WriteRay R = train_write_ray(i, ds, st, counts, base, ray_index, rays_out, rays_rgba, numsteps_out);
+	const WriteRay R = train_write_ray(ray_index[i], ds, st, counts[i], base[i], rays_out, rays_rgba, numsteps_out);
 	const uint32_t cap = train_write_cap(P, R.numsteps);
 	if (log.bits && st.logged) {
-		train_write_replay(i, P, st, cap, log, [&](uint32_t j, float t) {
-			train_write_sample(P, R.o, R.d, R.wdir, t, (size_t)R.base + j, coords_out, sink);
-			return true;
-		});
+		const ShortForm f = disparity_short_form(P);
+		uint32_t j = 0;
+		for (uint32_t w = 0; w < log.words; ++w)
+			if ((st.word_mask[w >> 5] >> (w & 31u)) & 1u)
+				train_replay_word(P, f, log.bits[(size_t)w * log.stride + i], log.t0[(size_t)w * log.stride + i], j, cap, [&](uint32_t k, float t) {
+					train_write_sample(P, R.o, R.d, R.wdir, t, (size_t)R.base + k, coords_out, sink);
+				});
 		return;
 	}
 	train_write_march(P, bitfield, R, cap, coords_out, sink);

@@ -30,6 +30,7 @@ __global__ void __launch_bounds__(RAY_CHUNK_BINS) k_ray_order(Params P, CountArg
 	const uint32_t n = A.n_rays - first < RAY_CHUNK ? A.n_rays - first : RAY_CHUNK;
 	const uint32_t chunk_image = train_ray_image(first, A);
 	bins[threadIdx.x] = 0;
+	if (blockIdx.x == 0 && threadIdx.x == 0 && A.parked_count) *A.parked_count = 0u;      // the queue of the counting march that follows
 	__syncthreads();
 	for (uint32_t j = threadIdx.x; j < n; j += RAY_CHUNK_BINS) {
 		const uint32_t k = ray_chunk_key_body(first + j, chunk_image, P, A);
@@ -155,25 +156,25 @@ __global__ void __launch_bounds__(128) k_train_count_wide(Params P, CountArgs A)
 	}
 }
 
-__global__ void k_zero_word(uint32_t* p) { *p = 0u; }
-
-// Sample offsets and ray indices of a training batch in three launches.  A ray's first sample is the sum of the counts of
-// all rays before it (occupancy_sampler.cu:634: the counter advances by every ray's count, kept or not); a ray is kept when
-// its samples fit (train_keep_flag); a kept ray's index is the number of kept rays before it.  Tiles of 1024 rays:
+// Sample offsets, ray indices and the list of write entries of a training batch in three launches.  A ray's first sample is the sum
+// of the counts of all rays before it (occupancy_sampler.cu:634: the counter advances by every ray's count, kept or not); a ray is
+// kept when its samples fit (train_keep_flag); a kept ray's index is the number of kept rays before it.  Tiles of 1024 rays:
 //   k_train_tile_counts   count sum of every tile; copies the two counters' values at entry
 //   k_train_bases         a tile's first offset = entry value + the sums of the tiles before it (every workgroup adds them up
-//                         itself: 1024 words for 2^20 rays); offsets, keep flags, kept rays of the tile; new sample counter
-//   k_train_ray_indices   the same over the kept flags; new ray counter
+//                         itself: 1024 words for 2^20 rays); offsets, kept rays and entries of the tile; new sample counter
+//   k_train_rays          the same over the kept rays and over their entries: what the kept rays themselves write, their
+//                         entries, the new ray counter
 constexpr uint32_t OFFSET_THREADS = 256;
 constexpr uint32_t OFFSET_TILE = 1024;
 
 struct TrainOffsetScratch {
 	uint32_t* tile_counts;   // [n_tiles]
 	uint32_t* tile_kept;     // [n_tiles]
-	uint32_t* entry;         // [2]: sample counter, ray counter when the call began
+	uint32_t* tile_entries;  // [n_tiles]
+	uint32_t* entry;         // [2]: sample counter, ray counter when the call began; [2]: write entries of the batch
 };
 
-static size_t train_offset_scratch_bytes(uint32_t n_rays) { return align_up(((size_t)div_up(n_rays ? n_rays : 1u, OFFSET_TILE) * 2 + 2) * sizeof(uint32_t), 256); }
+static size_t train_offset_scratch_bytes(uint32_t n_rays) { return align_up(((size_t)div_up(n_rays ? n_rays : 1u, OFFSET_TILE) * 3 + 3) * sizeof(uint32_t), 256); }
 
 __global__ void __launch_bounds__(OFFSET_THREADS) k_train_tile_counts(uint32_t n_rays, const uint32_t* __restrict__ counts, TrainOffsetScratch S,
                                                                       const uint32_t* __restrict__ n_coords_counter, const uint32_t* __restrict__ n_rays_counter) {
@@ -187,122 +188,145 @@ __global__ void __launch_bounds__(OFFSET_THREADS) k_train_tile_counts(uint32_t n
 }
 
 // sum of the tile sums before this workgroup's tile (wrapping, like the counter it continues)
+template <uint32_t THREADS>
 __device__ __forceinline__ uint32_t tiles_before(const uint32_t* __restrict__ tile_sums, uint32_t* lds) {
 	uint32_t v = 0;
-	for (uint32_t k = threadIdx.x; k < blockIdx.x; k += OFFSET_THREADS) v += tile_sums[k];
-	return block_sum_u32<OFFSET_THREADS>(v, lds);
+	for (uint32_t k = threadIdx.x; k < blockIdx.x; k += THREADS) v += tile_sums[k];
+	return block_sum_u32<THREADS>(v, lds);
 }
 
-__global__ void __launch_bounds__(OFFSET_THREADS) k_train_bases(uint32_t n_rays, uint32_t n_coords, const uint32_t* __restrict__ counts, TrainOffsetScratch S,
-                                                                uint32_t* __restrict__ base, uint32_t* __restrict__ keep, uint32_t* __restrict__ n_coords_counter) {
+__global__ void __launch_bounds__(OFFSET_THREADS) k_train_bases(uint32_t n_rays, uint32_t n_coords, const uint32_t* __restrict__ counts, const uint32_t* __restrict__ n_entries, TrainOffsetScratch S,
+                                                                uint32_t* __restrict__ base, uint32_t* __restrict__ n_coords_counter) {
 	__shared__ uint32_t lds[OFFSET_THREADS / 64 + 1];
-	const uint32_t before = S.entry[0] + tiles_before(S.tile_counts, lds);
+	const uint32_t before = S.entry[0] + tiles_before<OFFSET_THREADS>(S.tile_counts, lds);
 	const uint32_t first = blockIdx.x * OFFSET_TILE + threadIdx.x * 4;
 	uint32_t c[4];
 	uint32_t sum = 0;
 	for (uint32_t k = 0; k < 4; ++k) { c[k] = first + k < n_rays ? counts[first + k] : 0u; sum += c[k]; }
 	uint32_t total;
 	uint32_t run = before + block_exclusive_scan_u32<OFFSET_THREADS>(sum, lds, &total);
-	uint32_t kept = 0;
+	uint32_t kept = 0, entries = 0;
 	for (uint32_t k = 0; k < 4; ++k) {
 		if (first + k < n_rays) {
-			const uint32_t flag = train_keep_flag(c[k], run, n_coords);
 			base[first + k] = run;
-			keep[first + k] = flag;
-			kept += flag;
+			if (train_keep_flag(c[k], run, n_coords)) { ++kept; entries += n_entries[first + k]; }
 		}
 		run += c[k];
 	}
-	const uint32_t kept_total = block_sum_u32<OFFSET_THREADS>(kept, lds);
+	const uint32_t kept_total = block_sum_u32<OFFSET_THREADS>(kept, lds), entries_total = block_sum_u32<OFFSET_THREADS>(entries, lds);
 	if (threadIdx.x == 0) {
 		S.tile_kept[blockIdx.x] = kept_total;
+		S.tile_entries[blockIdx.x] = entries_total;
 		if (blockIdx.x + 1 == gridDim.x) *n_coords_counter = before + total;
 	}
 }
 
-__global__ void __launch_bounds__(OFFSET_THREADS) k_train_ray_indices(uint32_t n_rays, const uint32_t* __restrict__ keep, TrainOffsetScratch S,
-                                                                      uint32_t* __restrict__ ridx, uint32_t* __restrict__ n_rays_counter) {
-	__shared__ uint32_t lds[OFFSET_THREADS / 64 + 1];
-	const uint32_t before = S.entry[1] + tiles_before(S.tile_kept, lds);
-	const uint32_t first = blockIdx.x * OFFSET_TILE + threadIdx.x * 4;
-	uint32_t f[4];
-	uint32_t sum = 0;
-	for (uint32_t k = 0; k < 4; ++k) { f[k] = first + k < n_rays ? keep[first + k] : 0u; sum += f[k]; }
-	uint32_t total;
-	uint32_t run = before + block_exclusive_scan_u32<OFFSET_THREADS>(sum, lds, &total);
-	for (uint32_t k = 0; k < 4; ++k) {
-		if (first + k < n_rays) ridx[first + k] = run;
-		run += f[k];
+// One thread a ray: a batch of a few thousand rays has sixty entries each while its grid is still full.
+__global__ void __launch_bounds__(OFFSET_TILE) k_train_rays(uint32_t n_rays, uint32_t n_coords, DatasetArgs ds, const TrainRay* __restrict__ state, const uint32_t* __restrict__ counts,
+                                                            const uint32_t* __restrict__ base, const uint32_t* __restrict__ n_entries, TrainOffsetScratch S,
+                                                            float* __restrict__ rays_out, float* __restrict__ rays_rgba, uint32_t* __restrict__ numsteps_out,
+                                                            U2* __restrict__ entries, uint32_t entry_capacity, uint32_t* __restrict__ n_rays_counter) {
+	__shared__ uint32_t lds[OFFSET_TILE / 64 + 1];
+	const uint32_t rays_before = S.entry[1] + tiles_before<OFFSET_TILE>(S.tile_kept, lds);
+	const uint32_t entries_before = tiles_before<OFFSET_TILE>(S.tile_entries, lds);
+	const uint32_t i = blockIdx.x * OFFSET_TILE + threadIdx.x;
+	const uint32_t count = i < n_rays ? counts[i] : 0u, first = i < n_rays ? base[i] : 0u;
+	const bool kept = i < n_rays && train_keep_flag(count, first, n_coords) != 0u;
+	uint32_t total_kept, total_entries;
+	const uint32_t r = rays_before + block_exclusive_scan_u32<OFFSET_TILE>(kept ? 1u : 0u, lds, &total_kept);
+	uint32_t at = entries_before + block_exclusive_scan_u32<OFFSET_TILE>(kept ? n_entries[i] : 0u, lds, &total_entries);
+	if (threadIdx.x == 0 && blockIdx.x + 1 == gridDim.x) {
+		*n_rays_counter = rays_before + total_kept;
+		S.entry[2] = entries_before + total_entries;
 	}
-	if (threadIdx.x == 0 && blockIdx.x + 1 == gridDim.x) *n_rays_counter = before + total;
+	if (!kept) return;
+	const TrainRay st = state[i];
+	train_write_ray(r, ds, st, count, first, rays_out, rays_rgba, numsteps_out);
+	auto put = [&](uint32_t word, uint32_t rank) {
+		if (at < entry_capacity) { U2 e; e.x = i; e.y = word | (rank << 8); entries[at] = e; }
+		++at;
+	};
+	if (!st.logged) { put(ENTRY_MARCH, 0u); return; }
+	uint32_t rank = 0;
+	#pragma unroll
+	for (uint32_t g = 0; g < 3; ++g)
+		for (uint32_t m = st.word_mask[g]; m; m &= m - 1u) put(g * 32u + (uint32_t)__builtin_ctz(m), rank++);
 }
 
-// Writing march, one wavefront per block.  The samples of the block's kept rays form one run of the sample arrays
-// (offsets are in ray order).  The run goes through LDS in windows: each lane replays its ray's step log, which only
-// yields the t of every sample, and drops t and its own number into the sample's slot; then consecutive lanes take
-// consecutive slots, compute what the sample stores (warp, cell, step) and write it, so that the per-sample work
-// is spread evenly whatever the rays' sample counts are, and the stores of a wavefront are contiguous.
+// Writing march, one wavefront per block, 64 entries at a time.  Every lane replays one log word (at most 32 steps of the t chain) and
+// drops the samples' t and its own number into LDS; then consecutive lanes take consecutive samples, compute what a sample
+// stores (warp, cell, step) and write it, so that the per-sample work is spread evenly and the stores of a wavefront are contiguous.
+// Bound by the per-sample work's vector instructions (some 200 a sample).  Handing out entries instead of 64 rays a wavefront is what makes
+// the time follow the number of samples: 4096 rays of a thousand samples each 39.6 ms -> 60 us, 2^20 rays of 15 samples 189 us -> 140 us
+// (a wavefront of 64 such long rays had 66 windows of samples to itself, and replayed each ray's log from its beginning for every one).
 constexpr uint32_t WRITE_WINDOW = 1024;
+constexpr uint32_t WRITE_WAVES = 8192;      // wavefronts of the launch: 32 a CU, more than are resident at once
 
-struct WindowEmit {
-	float* win_t; uint8_t* win_ray;
-	uint32_t first, size, base, lane;      // window [first, first + size) of sample indices; the ray's first sample
-	__device__ bool operator()(uint32_t j, float t) const {
-		const uint32_t k = base + j;
-		if (k >= first + size) return false;               // the rest of the ray belongs to later windows
-		if (k >= first) { win_t[k - first] = t; win_ray[k - first] = (uint8_t)lane; }
-		return true;
-	}
-};
-
-__global__ void __launch_bounds__(64) k_train_write(Params P, uint32_t n_rays, DatasetArgs ds, const uint8_t* __restrict__ bitfield,
-                                                    const TrainRay* __restrict__ state, const uint32_t* __restrict__ counts,
-                                                    const uint32_t* __restrict__ base, const uint32_t* __restrict__ keep,
-                                                    const uint32_t* __restrict__ ray_index,
-                                                    float* __restrict__ rays_out, float* __restrict__ rays_rgba, uint32_t* __restrict__ numsteps_out,
+__global__ void __launch_bounds__(64) k_train_write(Params P, const uint8_t* __restrict__ bitfield, const TrainRay* __restrict__ state, const uint32_t* __restrict__ counts,
+                                                    const uint32_t* __restrict__ base, const U2* __restrict__ entries, const uint32_t* __restrict__ n_entries, uint32_t entry_capacity,
                                                     float* __restrict__ coords_out, float* __restrict__ sample_t, float* __restrict__ sample_dt, uint32_t* __restrict__ sample_cell, StepLog log) {
 	__shared__ float win_t[WRITE_WINDOW];
-	__shared__ uint8_t win_ray[WRITE_WINDOW];
-	__shared__ float ray_odw[64][9];             // origin, direction, warped direction of the lanes' rays
+	__shared__ uint8_t win_lane[WRITE_WINDOW];
+	__shared__ float ray_od[64][7];              // origin and direction of the lanes' rays (an odd stride: no two lanes on one bank)
+	__shared__ uint32_t place[64];               // where a lane's samples go, minus their position among the wavefront's samples
 	const uint32_t lane = threadIdx.x;
-	const uint32_t i = (gridDim.x - 1u - blockIdx.x) * 64u + lane;      // last rays first, like the counting march (181 -> 171 us)
-	const bool kept = i < n_rays && keep[i] != 0;
+	const uint32_t listed = *n_entries, n = listed < entry_capacity ? listed : entry_capacity;
+	const ShortForm f = disparity_short_form(P);
 	DirectSink out;
 	out.sample_t = sample_t; out.sample_dt = sample_dt; out.sample_cell = sample_cell;
-	TrainRay st;
-	WriteRay R;
-	R.numsteps = 0; R.base = 0;
-	bool replayed = false;
-	if (kept) {
-		st = state[i];
-		R = train_write_ray(i, ds, st, counts, base, ray_index, rays_out, rays_rgba, numsteps_out);
-		st3(&ray_odw[lane][0], R.o); st3(&ray_odw[lane][3], R.d); st3(&ray_odw[lane][6], R.wdir);
-		replayed = log.bits != nullptr && st.logged != 0u;
-		// without a usable log the ray marches again on its own
-		if (!replayed) train_write_march(P, bitfield, R, train_write_cap(P, R.numsteps), coords_out, out);
-	}
-	// the block's run of replayed samples
-	uint32_t lo = replayed ? R.base : 0xffffffffu, hi = replayed ? R.base + R.numsteps : 0u;
-	for (uint32_t off = 32; off > 0; off >>= 1) {
-		const uint32_t lo2 = (uint32_t)__shfl_xor((int)lo, (int)off, 64), hi2 = (uint32_t)__shfl_xor((int)hi, (int)off, 64);
-		lo = lo2 < lo ? lo2 : lo;
-		hi = hi2 > hi ? hi2 : hi;
-	}
-	for (uint32_t first = lo; first < hi; first += WRITE_WINDOW) {     // uniform: lo and hi are the same in every lane
-		const uint32_t size = hi - first < WRITE_WINDOW ? hi - first : WRITE_WINDOW;
-		for (uint32_t q = lane; q < size; q += 64u) win_t[q] = srf_u2f(WINDOW_EMPTY);
-		__syncthreads();
-		if (replayed && R.base < first + size && R.base + R.numsteps > first) {
-			WindowEmit emit;
-			emit.win_t = win_t; emit.win_ray = win_ray; emit.first = first; emit.size = size; emit.base = R.base; emit.lane = lane;
-			train_write_replay(i, P, st, train_write_cap(P, R.numsteps), log, emit);
+	for (uint64_t first = (uint64_t)blockIdx.x * 64u; first < n; first += (uint64_t)gridDim.x * 64u) {
+		const bool mine = first + lane < n;
+		U2 e; e.x = 0u; e.y = ENTRY_MARCH;
+		if (mine) e = entries[first + lane];
+		const uint32_t i = e.x, word = e.y & 0xffu, rank = e.y >> 8;
+		const bool marches = word == ENTRY_MARCH;
+		uint32_t bits = 0u, ray_base = 0u;
+		float t0 = 0.f;
+		Vec3 o = mk3(0.f, 0.f, 0.f), d = o;
+		if (mine) {
+			ray_base = base[i];
+			if (!marches) { bits = log.bits[(size_t)word * log.stride + i]; t0 = log.t0[(size_t)word * log.stride + i]; }
+			o = ld3(state[i].o); d = ld3(state[i].d);
 		}
-		__syncthreads();
-		for (uint32_t q = lane; q < size; q += 64u) {
-			const float t = win_t[q];
-			if (srf_f2u(t) == WINDOW_EMPTY) continue;      // a slot of a ray that was dropped or has marched on its own
-			const float* r = ray_odw[win_ray[q]];
-			train_write_sample(P, ld3(r), ld3(r + 3), ld3(r + 6), t, (size_t)first + q, coords_out, out);
+		// the first entry's ray may have begun before it: its samples so far are those of its earlier words
+		uint32_t carry = 0u;
+		const uint32_t rank0 = lane_value_u32(rank, 0u);
+		if (rank0 != 0u) {
+			const uint32_t i0 = lane_value_u32(i, 0u), word0 = lane_value_u32(word, 0u);
+			for (uint32_t w = lane; w < word0; w += 64u)
+				if ((state[i0].word_mask[w >> 5] >> (w & 31u)) & 1u) carry += (uint32_t)__popc(log.bits[(size_t)w * log.stride + i0]);
+			carry = wave_sum_fast(carry);
+		}
+		const uint32_t count = (uint32_t)__popc(bits);
+		const uint32_t incl = wave_inclusive_scan_fast(count), excl = incl - count;
+		// the sample before which the lane's ray has its first entry of this round
+		const uint32_t head = rank <= lane ? lane - rank : 0u;
+		const uint32_t ray_excl = (uint32_t)__shfl((int)excl, (int)head, 64);
+		place[lane] = ray_base + (rank > lane ? carry : 0u) - ray_excl;
+		st3(&ray_od[lane][0], o); st3(&ray_od[lane][3], d);
+		// a ray without a usable log marches again on its own
+		if (mine && marches) {
+			WriteRay R;
+			R.o = o; R.d = d; R.wdir = warp_direction(d); R.numsteps = counts[i]; R.base = ray_base; R.startt = state[i].startt;
+			train_write_march(P, bitfield, R, train_write_cap(P, R.numsteps), coords_out, out);
+		}
+		const uint32_t total = lane_value_u32(incl, 63u);
+		for (uint32_t lo = 0; lo < total;) {      // uniform: as many lanes' samples at a time as fit the window
+			const bool now = count != 0u && excl >= lo && incl - lo <= WRITE_WINDOW;
+			const uint32_t size = wave_max_fast(now ? incl - lo : 0u);
+			__syncthreads();
+			if (now) {
+				uint32_t j = 0;
+				train_replay_word(P, f, bits, t0, j, 32u, [&](uint32_t k, float t) { win_t[excl - lo + k] = t; win_lane[excl - lo + k] = (uint8_t)lane; });
+			}
+			__syncthreads();
+			for (uint32_t q = lane; q < size; q += 64u) {
+				const uint32_t l = win_lane[q];
+				const float* r = ray_od[l];
+				const Vec3 rd = ld3(r + 3);
+				train_write_sample(P, ld3(r), rd, warp_direction(rd), win_t[q], (size_t)(uint32_t)(place[l] + lo + q), coords_out, out);
+			}
+			lo += size;
 		}
 		__syncthreads();
 	}
@@ -571,9 +595,8 @@ int srf_sampler_sample_coords_from_dataset(srf_sampler_t* s, uint32_t n_rays, ui
 	const size_t off_state = 0;
 	const size_t off_counts = align_up(off_state + n * sizeof(TrainRay), 256);
 	const size_t off_base = align_up(off_counts + n * 4, 256);
-	const size_t off_keep = align_up(off_base + n * 4, 256);
-	const size_t off_ridx = align_up(off_keep + n * 4, 256);
-	const size_t off_scan = align_up(off_ridx + n * 4, 256);
+	const size_t off_n_entries = align_up(off_base + n * 4, 256);
+	const size_t off_scan = align_up(off_n_entries + n * 4, 256);
 	// step log: enough words for the marching-step bound of disparity stepping (n_max_steps plus start jitter and the
 	// final clamp to the far plane); rays that take more steps fall back to a full second march
 	uint32_t log_words = s->P.use_grid ? (s->P.n_max_steps + 64 + 31) / 32 : 0;
@@ -587,14 +610,21 @@ int srf_sampler_sample_coords_from_dataset(srf_sampler_t* s, uint32_t n_rays, ui
 	const uint32_t parked_capacity = probe_budget ? (n_rays / 8u > 4096u ? n_rays / 8u : 4096u) : 0u;
 	const size_t off_parked = align_up(off_order + (sort_rays ? n * 4 : 0), 256);
 	const size_t off_parked_count = align_up(off_parked + (size_t)parked_capacity * sizeof(ParkedRay), 256);
-	rc = s->ws.reserve(off_parked_count + 256);
+	// write entries: as many as log words, and no more than kept samples (kept rays' samples fit below n_coords, unless the batch's sum of
+	// counts can wrap), one at least for every ray where nothing is logged
+	const uint64_t most_words = (uint64_t)n_rays * (log_words ? log_words : 1u);
+	const bool wraps = (uint64_t)n_rays * s->P.n_max_steps > 0xffffffffull;
+	const uint64_t most_entries = wraps || most_words < n_coords ? most_words : n_coords;
+	const uint32_t entry_capacity = most_entries > 0xffffffffull ? 0xffffffffu : (uint32_t)most_entries;
+	const size_t off_entries = align_up(off_parked_count + 256, 256);
+	rc = s->ws.reserve(off_entries + (size_t)entry_capacity * sizeof(U2) + 256);
 	if (rc != SRF_OK) return rc;
 	char* w = (char*)s->ws.ptr;
 	TrainRay* state = (TrainRay*)(w + off_state);
 	uint32_t* counts = (uint32_t*)(w + off_counts);
 	uint32_t* base = (uint32_t*)(w + off_base);
-	uint32_t* keep = (uint32_t*)(w + off_keep);
-	uint32_t* ridx = (uint32_t*)(w + off_ridx);
+	uint32_t* n_entries = (uint32_t*)(w + off_n_entries);
+	U2* entries = (U2*)(w + off_entries);
 	void* scan = w + off_scan;
 	StepLog log;
 	log.bits = log_words ? (uint32_t*)(w + off_log) : nullptr;
@@ -611,14 +641,13 @@ int srf_sampler_sample_coords_from_dataset(srf_sampler_t* s, uint32_t n_rays, ui
 
 	CountArgs ca;
 	ca.n_rays = n_rays; ca.n_rays_shift = n_rays_shift; ca.ds = ds; ca.bitfield = bitfield; ca.rng = r;
-	ca.state = state; ca.counts = counts; ca.log = log;
+	ca.state = state; ca.counts = counts; ca.n_entries = n_entries; ca.log = log;
 	ca.skip = sampler_skip_table(s);
 	ca.probe_budget = probe_budget;
 	ca.park_lanes = s->count_park_lanes;
 	ca.parked = (ParkedRay*)(w + off_parked);
 	ca.parked_capacity = parked_capacity;
 	ca.parked_count = (uint32_t*)(w + off_parked_count);
-	if (probe_budget) hipLaunchKernelGGL(k_zero_word, dim3(1), dim3(1), 0, st, ca.parked_count);
 	// rays per wavefront: enough for lanes that finish early to pick up more work, few enough for several wavefronts per SIMD
 	// (settled by measurement on the 2^20-ray training batch: one ray a lane; a probe round once every lane waits for one or the stepping
 	// lanes are outnumbered 32 to 1 — 4: 1.52, 8: 1.41, 16: 1.33, 24: 1.30, 32: 1.29, 48: 1.31, 64: 1.37 ms; stepping rounds are cheap since
@@ -679,14 +708,16 @@ int srf_sampler_sample_coords_from_dataset(srf_sampler_t* s, uint32_t n_rays, ui
 	}
 	const uint32_t n_tiles = div_up(n_rays, OFFSET_TILE);
 	TrainOffsetScratch os;
-	os.tile_counts = (uint32_t*)scan; os.tile_kept = os.tile_counts + n_tiles; os.entry = os.tile_kept + n_tiles;
+	os.tile_counts = (uint32_t*)scan; os.tile_kept = os.tile_counts + n_tiles; os.tile_entries = os.tile_kept + n_tiles; os.entry = os.tile_entries + n_tiles;
 	hipLaunchKernelGGL(k_train_tile_counts, dim3(n_tiles), dim3(OFFSET_THREADS), 0, st, n_rays, (const uint32_t*)counts, os, (const uint32_t*)n_coords_counter, (const uint32_t*)n_rays_counter);
-	hipLaunchKernelGGL(k_train_bases, dim3(n_tiles), dim3(OFFSET_THREADS), 0, st, n_rays, n_coords, (const uint32_t*)counts, os, base, keep, n_coords_counter);
-	hipLaunchKernelGGL(k_train_ray_indices, dim3(n_tiles), dim3(OFFSET_THREADS), 0, st, n_rays, (const uint32_t*)keep, os, ridx, n_rays_counter);
+	hipLaunchKernelGGL(k_train_bases, dim3(n_tiles), dim3(OFFSET_THREADS), 0, st, n_rays, n_coords, (const uint32_t*)counts, (const uint32_t*)n_entries, os, base, n_coords_counter);
+	hipLaunchKernelGGL(k_train_rays, dim3(n_tiles), dim3(OFFSET_TILE), 0, st, n_rays, n_coords, ds, (const TrainRay*)state, (const uint32_t*)counts, (const uint32_t*)base,
+	                   (const uint32_t*)n_entries, os, rays, rays_rgba, ray_coord_indices, entries, entry_capacity, n_rays_counter);
 	SRF_LAUNCH_CHECK();
-	hipLaunchKernelGGL(k_train_write, dim3(div_up(n_rays, 64)), dim3(64), 0, st, s->P, n_rays, ds, bitfield, (const TrainRay*)state,
-	                   (const uint32_t*)counts, (const uint32_t*)base, (const uint32_t*)keep, (const uint32_t*)ridx,
-	                   rays, rays_rgba, ray_coord_indices, coords, sample_t, sample_dt, sample_cell, log);
+	const uint32_t most_rounds = entry_capacity / 64u + (entry_capacity % 64u ? 1u : 0u);
+	if (most_rounds)
+		hipLaunchKernelGGL(k_train_write, dim3(most_rounds < WRITE_WAVES ? most_rounds : WRITE_WAVES), dim3(64), 0, st, s->P, bitfield, (const TrainRay*)state, (const uint32_t*)counts,
+		                   (const uint32_t*)base, (const U2*)entries, (const uint32_t*)(os.entry + 2), entry_capacity, coords, sample_t, sample_dt, sample_cell, log);
 	SRF_LAUNCH_CHECK();
 	return SRF_OK;
 }
