@@ -276,9 +276,8 @@ SRF_HD void grid_sample_body(uint32_t i, const Params& P, uint32_t n_elements, P
 // in lockstep; the order in which phases run never changes what a ray computes.
 enum : uint32_t { LANE_IDLE = 0, LANE_PROBE = 1, LANE_STEP = 2 };
 
-// A ray that has used up its probe budget in the lane-per-ray march is parked here, as it stands, and finished by a
-// whole wavefront (wide_* below): rays that need a lookup at nearly every step would otherwise keep one lane, and with
-// it the wavefront, busy for thousands of memory round trips.
+// A ray that has used up its probe budget can be parked here, as it stands, and carried on 64 steps at a time (wide_* below).  The
+// kernels gather such rays in place instead (teams of lanes, srf_march.hip); the host build rehearses the same bookkeeping this way.
 struct ParkedRay {
 	uint32_t i, img, j, step, word, cur_w, logged;
 	uint32_t mask[3];
@@ -684,10 +683,14 @@ SRF_HD WideLookup wide_lookup(const Params& P, const CountArgs& A, Vec3 o, Vec3 
 SRF_HD uint32_t wide_flags(const WideLookup& q) { return !q.inside ? 0u : (((q.byte >> q.bit) & 1u) ? 3u : 1u); }
 SRF_HD uint32_t wide_probe(const Params& P, const CountArgs& A, Vec3 o, Vec3 d, float t) { return wide_flags(wide_lookup(P, A, o, d, t)); }
 
-SRF_HD void wide_apply(CountLane& L, const Params& P, const CountArgs& A, const float* t, uint64_t m_inside, uint64_t m_occ, uint64_t m_zero) {
+// The loop's bookkeeping for the next n_steps steps (at most 64), whose lookups are in: bit k of the masks is step k's, t[k] the t it
+// starts from, t_end the t behind the last.
+template <class Starts>
+SRF_HD void steps_apply(CountLane& L, const Params& P, const CountArgs& A, uint32_t n_steps, const Starts& t, float t_end, uint64_t m_inside, uint64_t m_occ, uint64_t m_zero) {
 	// the loop runs while the position is inside the box and the sample count is below the cap (occupancy_sampler.cu:595-597)
-	uint32_t n = ~m_inside ? (uint32_t)__builtin_ctzll(~m_inside) : WIDE_STEPS;
-	bool ended = n < WIDE_STEPS;
+	const uint64_t m_outside = ~m_inside & low_bits64(n_steps);
+	uint32_t n = m_outside ? (uint32_t)__builtin_ctzll(m_outside) : n_steps;
+	bool ended = n < n_steps;
 	const uint32_t allowed = L.j < P.n_max_steps ? P.n_max_steps - L.j : 0u;
 	if (!allowed) { n = 0; ended = true; }
 	else if ((uint32_t)__builtin_popcountll(m_occ & low_bits64(n)) >= allowed) {
@@ -695,7 +698,7 @@ SRF_HD void wide_apply(CountLane& L, const Params& P, const CountArgs& A, const 
 		uint64_t m = m_occ & low_bits64(n);
 		for (uint32_t a = 1; a < allowed; ++a) m &= m - 1ull;
 		const uint32_t last = (uint32_t)__builtin_ctzll(m) + 1u;
-		if (last < WIDE_STEPS) { n = last; ended = true; }
+		if (last < n_steps) { n = last; ended = true; }
 	}
 	// a step of size zero is taken and ends the march (count_advance)
 	const uint64_t z = m_zero & low_bits64(n);
@@ -718,8 +721,11 @@ SRF_HD void wide_apply(CountLane& L, const Params& P, const CountArgs& A, const 
 		rest &= ~in_word;
 	}
 	L.step += n;
-	L.t = L.t_limit = t[n];
+	L.t = L.t_limit = n < n_steps ? t[n] : t_end;
 	if (ended) count_finish(L, A);
+}
+SRF_HD void wide_apply(CountLane& L, const Params& P, const CountArgs& A, const float* t, uint64_t m_inside, uint64_t m_occ, uint64_t m_zero) {
+	steps_apply(L, P, A, WIDE_STEPS, t, t[WIDE_STEPS], m_inside, m_occ, m_zero);
 }
 
 // one parked ray from where it stopped to its end, the lanes' work done one after the other

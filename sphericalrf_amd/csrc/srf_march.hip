@@ -8,15 +8,19 @@
 
 namespace srf {
 
-// Counting march, one wavefront per block.  Each lane carries one ray through the phases of
-// srf_bodies.h's state machine; every round the wavefront runs the phase most of its lanes are
-// waiting for (stepping through known-empty space, probing the grid, or picking up the next ray
-// of the block's range), so the expensive probe is issued for many lanes at once instead of
-// whenever any single lane needs one.
+// Counting march, one wavefront per block.  Lanes carry rays through the phases of srf_bodies.h's state machine; every round the
+// wavefront runs one phase for the lanes that wait for it (stepping through known-empty space, or probing the grid), so the
+// expensive probe is issued for many lanes at once instead of whenever any single lane needs one.
+// Bound by vector instructions where there are rays enough (2^20 rays: 16384 wavefronts), by the round trips of a ray's probes one
+// after the other where there are not.  Rays are therefore worked on by teams of lanes: a batch of few rays begins with several
+// lanes a ray (see the launch), and a wavefront whose rays left fill half of its lanes at most gathers them and gives each twice the
+// lanes, up to a whole wavefront for the last one.  A team takes a ray through as many steps a round as it has lanes.  Against one lane
+// a ray with the rays that crawl finished by a second launch: 4096 rays of a thousand samples 3.58 + 0.08 ms -> 0.22 ms, 80 k rays 488 +
+// 48 us -> 290 us, 2^20 rays 1057 + 72 us -> 985 us.
 // steps per stepping round, at most: long enough to spread the round's fixed work (phase ballots, the first reciprocal of the
 // chain, the closed-form stretch) over many steps; the burst runs in groups of four and ends when no lane has a step left, so a
 // long limit costs the lanes that wait for a probe little (24: 1.51 ms, 32: 1.33 ms, 48: 1.29 ms, 64: 1.35 ms for the march of
-// the 2^20-ray batch, with probing lanes waiting until they outnumber the stepping ones 32 to 1)
+// the 2^20-ray batch)
 constexpr uint32_t COUNT_STEP_BURST = 48;
 
 // five wavefronts a SIMD: 102 registers a lane, which the counting march just fits
@@ -30,7 +34,6 @@ __global__ void __launch_bounds__(RAY_CHUNK_BINS) k_ray_order(Params P, CountArg
 	const uint32_t n = A.n_rays - first < RAY_CHUNK ? A.n_rays - first : RAY_CHUNK;
 	const uint32_t chunk_image = train_ray_image(first, A);
 	bins[threadIdx.x] = 0;
-	if (blockIdx.x == 0 && threadIdx.x == 0 && A.parked_count) *A.parked_count = 0u;      // the queue of the counting march that follows
 	__syncthreads();
 	for (uint32_t j = threadIdx.x; j < n; j += RAY_CHUNK_BINS) {
 		const uint32_t k = ray_chunk_key_body(first + j, chunk_image, P, A);
@@ -52,9 +55,88 @@ __global__ void __launch_bounds__(RAY_CHUNK_BINS) k_ray_order(Params P, CountArg
 	for (uint32_t j = threadIdx.x; j < n; j += RAY_CHUNK_BINS) order[first + atomicAdd(&bins[keys[j]], 1u)] = first + j;
 }
 
+// A team of lanes takes one ray through its next `team` steps at once: the step sizes do not depend on what the grid holds
+// (occupancy_sampler.cu:629-632: t += dt whatever the cell), so every lane follows the chain of t, keeps the start of the step that
+// is its own, and looks that position up; the loop's bookkeeping is then replayed over the team's results in step order.  How far
+// nothing can be found behind those steps is what the last of them says.  All lanes of a team hold the same state of their ray.
 template <bool SPHERE>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(SRF_COUNT_WAVES_PER_EU))) k_train_count(Params P, CountArgs A, uint32_t rays_per_wave, uint32_t probe_quorum, uint32_t begin_quorum, uint32_t probe_ratio,
-                                                                                                                    const uint32_t* __restrict__ order, unsigned long long* timing) {
+__device__ __forceinline__ void count_team_probe(CountLane& L, const Params& P, const CountArgs& A, uint32_t team, float* starts) {
+	const uint32_t lane = threadIdx.x & 63u, sub = lane & (team - 1u), lead = lane - sub;
+	const float cone = P.cone_angle_constant;
+	const bool mine = L.phase == LANE_PROBE;
+	const ShortForm f = disparity_short_form(P);
+	const bool chains = f.usable && L.t >= f.t_lo;
+	ShortChain ch = short_chain_at(chains ? L.t : 1.f);
+	float t_mine = L.t;
+	for (uint32_t k = 0; k < team; ++k) {
+		t_mine = k == sub ? ch.t : t_mine;
+		ch = short_chain_next(f, ch);
+	}
+	float t_end = ch.t;
+	bool zero = false;
+	const uint64_t own = low_bits64(team) << lead;
+	// every step has to start inside the short form's range; a team with one that does not goes through calc_dt
+	const uint64_t outside_form = __ballot(!chains || !(t_mine >= f.t_lo && t_mine <= f.t_hi));
+	if (mine && (outside_form & own) != 0ull) {
+		float t = L.t;
+		for (uint32_t k = 0; k < team; ++k) {
+			const float dt = calc_dt(P, t, cone);
+			if (k == sub) { t_mine = t; zero = dt == 0.f; }
+			t += dt;
+		}
+		t_end = t;
+	}
+	bool inside = false, occupied = false;
+	float limit = t_mine;
+	if (mine) {
+		const Vec3 pos = along(L.o, L.d, t_mine);
+		inside = aabb_contains(P, pos);
+		bool look = inside;
+		if (SPHERE && inside && P.sphere[3] > 0.f) {
+			float t_enter;
+			const SphereGate g = sphere_gate(P, L.o, L.d, t_mine, &t_enter);
+			if (g == SPHERE_BEYOND) inside = look = false;
+			if (g == SPHERE_BEFORE) { look = false; limit = t_enter; }
+		}
+		if (look) {
+			const Probe s = probe_at(P, P.use_grid ? A.bitfield : nullptr, pos, t_mine, cone, &A.skip);
+			occupied = s.occ;
+			if (!occupied && A.skip.dist != nullptr && P.use_grid) limit = skip_limit(P, A.skip, L.sr, L.o, L.d, t_mine, s.radius, s.level);
+		}
+	}
+	const uint64_t m_inside = __ballot(inside) >> lead, m_occ = __ballot(occupied) >> lead, m_zero = __ballot(zero) >> lead;
+	starts[lane] = t_mine;
+	limit = __shfl(limit, (int)(lead + team - 1u), 64);
+	__syncthreads();
+	if (mine) {
+		steps_apply(L, P, A, team, starts + lead, t_end, m_inside, m_occ & low_bits64(team), m_zero);
+		if (L.phase != LANE_IDLE) {
+			L.t_limit = limit;
+			L.phase = L.t < L.t_limit ? LANE_STEP : LANE_PROBE;
+		}
+	}
+	__syncthreads();
+}
+
+__device__ __forceinline__ float moved(float v, uint32_t from) { return __shfl(v, (int)from, 64); }
+__device__ __forceinline__ uint32_t moved(uint32_t v, uint32_t from) { return (uint32_t)__shfl((int)v, (int)from, 64); }
+__device__ __forceinline__ Vec3 moved(Vec3 v, uint32_t from) { return mk3(moved(v.x, from), moved(v.y, from), moved(v.z, from)); }
+// the state of the ray in lane `from`
+__device__ __forceinline__ void count_move(CountLane& L, uint32_t from) {
+	L.phase = moved(L.phase, from); L.i = moved(L.i, from); L.o = moved(L.o, from); L.d = moved(L.d, from);
+	L.t = moved(L.t, from); L.t_limit = moved(L.t_limit, from); L.t_word = moved(L.t_word, from); L.startt = moved(L.startt, from);
+	L.xy[0] = moved(L.xy[0], from); L.xy[1] = moved(L.xy[1], from);
+	L.img = moved(L.img, from); L.j = moved(L.j, from); L.step = moved(L.step, from); L.word = moved(L.word, from); L.cur_w = moved(L.cur_w, from);
+	for (int k = 0; k < 3; ++k) L.mask[k] = moved(L.mask[k], from);
+	L.logged = moved(L.logged ? 1u : 0u, from) != 0u;
+	L.sr = skip_ray_setup(L.o, L.d);
+}
+
+template <bool SPHERE>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(SRF_COUNT_WAVES_PER_EU))) k_train_count(Params P, CountArgs A, uint32_t team, uint32_t probe_ratio,
+                                                                                                                    const uint32_t* __restrict__ order) {
+	__shared__ float starts[64];
+	__shared__ uint32_t from_lane[64];
 	const uint32_t lane = threadIdx.x;
 	// The wavefronts are taken from the last rays of the batch to the first.  The kernel ends with its last wavefront, lifetimes
 	// differ by a factor of three between cameras, and how the expensive ones fall in the order of dispatch moves the kernel's time by
@@ -63,95 +145,41 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(SRF_COU
 	// first; several falling ramps; the cheapest quarter last; two or four runs of neighbouring chunks side by side) were all slower than
 	// the latter (presumably because whatever takes neighbouring cameras apart in time costs the lookups their locality); why the
 	// falling order beats the rising one in all three is not understood beyond that its last wavefronts happened to be cheap ones.
-	uint32_t next = (gridDim.x - 1u - blockIdx.x) * rays_per_wave;
-#ifdef SRF_KERNEL_TIMING
-	// per phase (step, probe, begin): cycles, rounds, lanes that took part
-	unsigned long long t_acc_[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-	unsigned long long t_prev_ = clock64();
-	const unsigned long long t_first_ = t_prev_, w_first_ = wall_clock64();
-#define SRF_COUNT_STAMP(k, lanes) do { const unsigned long long now_ = clock64(); t_acc_[k] += now_ - t_prev_; t_prev_ = now_; t_acc_[3 + k] += 1; t_acc_[6 + k] += (lanes); } while (0)
-#else
-#define SRF_COUNT_STAMP(k, lanes) ((void)0)
-#endif
-	const uint32_t end = next + rays_per_wave < A.n_rays ? next + rays_per_wave : A.n_rays;
+	const uint32_t at = (gridDim.x - 1u - blockIdx.x) * (64u / team) + lane / team;
 	CountLane L;
 	L.phase = LANE_IDLE;
+	if (at < A.n_rays) count_begin(L, order[at], P, A);
 	for (;;) {
-		const uint64_t m_idle = __ballot(L.phase == LANE_IDLE);
-		const uint32_t n_probe = (uint32_t)__popcll(__ballot(L.phase == LANE_PROBE));
-		const uint32_t n_step = (uint32_t)__popcll(__ballot(L.phase == LANE_STEP));
-		const uint32_t left = end - next;
-		uint32_t n_idle = (uint32_t)__popcll(m_idle);
-		n_idle = n_idle < left ? n_idle : left;
-		if (!(n_idle | n_probe | n_step)) break;
+		const uint64_t m_probe = __ballot(L.phase == LANE_PROBE), m_step = __ballot(L.phase == LANE_STEP);
+		const uint32_t n_probe = (uint32_t)__popcll(m_probe), n_step = (uint32_t)__popcll(m_step);
+		uint32_t alive = n_probe + n_step;
+		if (!alive) break;
+		if (alive <= 32u && team < 64u) {
+			// the rays left fill half of the lanes at most: they are gathered, and more lanes work on each
+			uint32_t larger = team;
+			while (alive * 2u <= 64u && larger < 64u) { larger *= 2u; alive *= 2u; }
+			const uint64_t m_alive = m_probe | m_step;
+			const bool leads = ((m_alive >> lane) & 1ull) != 0ull && (lane & (team - 1u)) == 0u;
+			const uint64_t m_lead = __ballot(leads);
+			if (leads) from_lane[__popcll(m_lead & ((1ull << lane) - 1ull))] = lane;
+			__syncthreads();
+			const uint32_t ray = lane / larger;
+			const bool takes = ray < (uint32_t)__popcll(m_lead);
+			const uint32_t from = takes ? from_lane[ray] : 0u;
+			count_move(L, from);
+			if (!takes) L.phase = LANE_IDLE;
+			team = larger;
+			__syncthreads();
+			continue;
+		}
 		// stepping is cheap and probing is not: lanes that want a probe wait while others step, until they are all of
 		// the wavefront or outnumber the stepping lanes probe_ratio to one (a few long skips must not hold up the rest)
-		const bool begin = n_idle >= begin_quorum || (n_idle && !n_probe && !n_step);
-		const bool step = !begin && n_step && n_probe < probe_quorum && n_probe < probe_ratio * n_step;
-		if (step) {
+		if (n_step && n_probe < probe_ratio * n_step) {
 			if (L.phase == LANE_STEP) count_steps<COUNT_STEP_BURST>(L, P, A);
-			SRF_COUNT_STAMP(0, n_step);
-		} else if (!begin) {
-			if (L.phase == LANE_PROBE) count_probe<SPHERE>(L, P, A, n_probe + n_step <= A.park_lanes);
-			SRF_COUNT_STAMP(1, n_probe);
+		} else if (team == 1u) {
+			if (L.phase == LANE_PROBE) count_probe<SPHERE>(L, P, A, false);
 		} else {
-			const uint32_t rank = (uint32_t)__popcll(m_idle & ((1ull << lane) - 1ull));
-			if (L.phase == LANE_IDLE && rank < n_idle) count_begin(L, order ? order[next + rank] : next + rank, P, A);
-			next += n_idle;
-			SRF_COUNT_STAMP(2, n_idle);
-		}
-	}
-#ifdef SRF_KERNEL_TIMING
-	if (lane == 0) {
-		for (int k = 0; k < 9; ++k) atomicAdd(&timing[(blockIdx.x & 1023u) * 16 + k], t_acc_[k]);
-		atomicAdd(&timing[(blockIdx.x & 1023u) * 16 + 9], clock64() - t_first_);
-		atomicAdd(&timing[(blockIdx.x & 1023u) * 16 + 10], wall_clock64() - w_first_);
-		const unsigned long long life_ = wall_clock64() - w_first_;
-		atomicMax(&timing[(blockIdx.x & 1023u) * 16 + 11], life_);
-		// histograms: lifetime in 100 us buckets, probe rounds in buckets of 64
-		const unsigned long long lb = life_ / 10000ull, pb = t_acc_[4] / 64ull;
-		atomicAdd(&timing[1024 * 16 + (lb < 47 ? lb : 47)], 1ull);
-		atomicAdd(&timing[1024 * 16 + 48 + (pb < 47 ? pb : 47)], 1ull);
-		const unsigned long long sb = t_acc_[3] / 64ull;
-		atomicAdd(&timing[1024 * 16 + 96 + (sb < 47 ? sb : 47)], 1ull);
-		// of the slow wavefronts (over 1 ms): step rounds, probe rounds, lanes per step round
-		if (life_ > 100000ull) { atomicAdd(&timing[1024 * 16 + 144], 1ull); atomicAdd(&timing[1024 * 16 + 145], t_acc_[3]); atomicAdd(&timing[1024 * 16 + 146], t_acc_[4]);
-			atomicAdd(&timing[1024 * 16 + 147], t_acc_[6]); atomicAdd(&timing[1024 * 16 + 148], t_acc_[7]); atomicAdd(&timing[1024 * 16 + 149], t_acc_[0]); atomicAdd(&timing[1024 * 16 + 150], t_acc_[1]); }
-	}
-#endif
-}
-
-// The wide march of the parked rays: one ray per workgroup of two wavefronts at a time.  The second wavefront runs the
-// chain of t one round (64 steps) ahead, since the step sizes do not depend on what the grid holds; in the first, every
-// lane looks one of the current round's 64 positions up and lane 0 replays the loop's bookkeeping over the results.
-template <bool SPHERE>
-__global__ void __launch_bounds__(128) k_train_count_wide(Params P, CountArgs A) {
-	__shared__ float t[2][WIDE_STEPS + 1];
-	__shared__ uint64_t zero_steps[2];
-	__shared__ uint32_t finished[2];      // per round parity, like t: a flag is not rewritten before both wavefronts have read it
-	const uint32_t lane = threadIdx.x & 63u;
-	const bool chain_wave = threadIdx.x >= 64u;
-	const uint32_t filled = *A.parked_count;
-	const uint32_t n = filled < A.parked_capacity ? filled : A.parked_capacity;
-	for (uint32_t q = blockIdx.x; q < n; q += gridDim.x) {
-		CountLane L;              // every lane has the ray (o and d are what the lookups need); lane 0 of the first wavefront advances it
-		count_unpark(L, A.parked[q]);
-		if (chain_wave && lane == 0) zero_steps[0] = wide_chain(P, L.t, t[0]);
-		__syncthreads();
-		for (uint32_t cur = 0;; cur ^= 1u) {
-			if (chain_wave) {
-				// the next round starts where this one ends, if the ray gets that far
-				if (lane == 0) zero_steps[cur ^ 1u] = wide_chain(P, t[cur][WIDE_STEPS], t[cur ^ 1u]);
-			} else {
-				const uint32_t f = wide_flags(wide_lookup<SPHERE>(P, A, L.o, L.d, t[cur][lane]));
-				const uint64_t m_inside = __ballot((f & 1u) != 0u), m_occ = __ballot((f & 2u) != 0u);
-				if (lane == 0) {
-					wide_apply(L, P, A, t[cur], m_inside, m_occ, zero_steps[cur]);
-					finished[cur] = L.phase == LANE_IDLE ? 1u : 0u;
-				}
-			}
-			__syncthreads();      // t[cur] and finished[cur] are rewritten in the round after next
-			if (finished[cur]) break;
+			count_team_probe<SPHERE>(L, P, A, team, starts);
 		}
 	}
 }
@@ -603,20 +631,14 @@ int srf_sampler_sample_coords_from_dataset(srf_sampler_t* s, uint32_t n_rays, ui
 	if (log_words > LOG_MAX_WORDS) log_words = LOG_MAX_WORDS;
 	const size_t off_log = align_up(off_scan + train_offset_scratch_bytes(n_rays), 256);
 	// marching order: chunks of rays sorted by (image, pixel tile)
-	constexpr bool sort_rays = true;
 	const size_t off_order = align_up(off_log + (size_t)log_words * n * 8, 256);
-	// rays that exhaust their probe budget are parked and finished by the wide march (0 = never)
-	const uint32_t probe_budget = s->count_probe_budget;
-	const uint32_t parked_capacity = probe_budget ? (n_rays / 8u > 4096u ? n_rays / 8u : 4096u) : 0u;
-	const size_t off_parked = align_up(off_order + (sort_rays ? n * 4 : 0), 256);
-	const size_t off_parked_count = align_up(off_parked + (size_t)parked_capacity * sizeof(ParkedRay), 256);
 	// write entries: as many as log words, and no more than kept samples (kept rays' samples fit below n_coords, unless the batch's sum of
 	// counts can wrap), one at least for every ray where nothing is logged
 	const uint64_t most_words = (uint64_t)n_rays * (log_words ? log_words : 1u);
 	const bool wraps = (uint64_t)n_rays * s->P.n_max_steps > 0xffffffffull;
 	const uint64_t most_entries = wraps || most_words < n_coords ? most_words : n_coords;
 	const uint32_t entry_capacity = most_entries > 0xffffffffull ? 0xffffffffu : (uint32_t)most_entries;
-	const size_t off_entries = align_up(off_parked_count + 256, 256);
+	const size_t off_entries = align_up(off_order + n * 4, 256);
 	rc = s->ws.reserve(off_entries + (size_t)entry_capacity * sizeof(U2) + 256);
 	if (rc != SRF_OK) return rc;
 	char* w = (char*)s->ws.ptr;
@@ -625,6 +647,7 @@ int srf_sampler_sample_coords_from_dataset(srf_sampler_t* s, uint32_t n_rays, ui
 	uint32_t* base = (uint32_t*)(w + off_base);
 	uint32_t* n_entries = (uint32_t*)(w + off_n_entries);
 	U2* entries = (U2*)(w + off_entries);
+	uint32_t* order = (uint32_t*)(w + off_order);
 	void* scan = w + off_scan;
 	StepLog log;
 	log.bits = log_words ? (uint32_t*)(w + off_log) : nullptr;
@@ -643,69 +666,23 @@ int srf_sampler_sample_coords_from_dataset(srf_sampler_t* s, uint32_t n_rays, ui
 	ca.n_rays = n_rays; ca.n_rays_shift = n_rays_shift; ca.ds = ds; ca.bitfield = bitfield; ca.rng = r;
 	ca.state = state; ca.counts = counts; ca.n_entries = n_entries; ca.log = log;
 	ca.skip = sampler_skip_table(s);
-	ca.probe_budget = probe_budget;
-	ca.park_lanes = s->count_park_lanes;
-	ca.parked = (ParkedRay*)(w + off_parked);
-	ca.parked_capacity = parked_capacity;
-	ca.parked_count = (uint32_t*)(w + off_parked_count);
-	// rays per wavefront: enough for lanes that finish early to pick up more work, few enough for several wavefronts per SIMD
-	// (settled by measurement on the 2^20-ray training batch: one ray a lane; a probe round once every lane waits for one or the stepping
-	// lanes are outnumbered 32 to 1 — 4: 1.52, 8: 1.41, 16: 1.33, 24: 1.30, 32: 1.29, 48: 1.31, 64: 1.37 ms; stepping rounds are cheap since
-	// whole stretches are taken in closed form, so the probes wait for nearly all of them; new rays are begun 32 at a time)
-	constexpr uint32_t rays_per_wave = 64, probe_quorum = 64, begin_quorum = 32, probe_ratio = 32;
-	const uint32_t* order = nullptr;
-	if (sort_rays) {
-		uint32_t* order_out = (uint32_t*)(w + off_order);
-		hipLaunchKernelGGL(k_ray_order, dim3(div_up(n_rays, RAY_CHUNK)), dim3(RAY_CHUNK_BINS), 0, st, s->P, ca, order_out);
-		SRF_LAUNCH_CHECK();
-		order = order_out;
-	}
-	unsigned long long* timing = nullptr;
-#ifdef SRF_KERNEL_TIMING
-	static unsigned long long* timing_buf = nullptr;
-	if (!timing_buf) { SRF_HIP(hipMalloc((void**)&timing_buf, (1024 * 16 + 192) * 8)); SRF_HIP(hipMemset(timing_buf, 0, (1024 * 16 + 192) * 8)); }
-	timing = timing_buf;
-#endif
-	if (s->P.sphere[3] > 0.f)
-		hipLaunchKernelGGL(k_train_count<true>, dim3(div_up(n_rays, rays_per_wave)), dim3(64), 0, st, s->P, ca, rays_per_wave, probe_quorum, begin_quorum, probe_ratio, order, timing);
-	else
-		hipLaunchKernelGGL(k_train_count<false>, dim3(div_up(n_rays, rays_per_wave)), dim3(64), 0, st, s->P, ca, rays_per_wave, probe_quorum, begin_quorum, probe_ratio, order, timing);
-#ifdef SRF_KERNEL_TIMING
-	{
-		static unsigned long long hs[1024 * 16 + 192];
-		unsigned long long h[12] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-		SRF_HIP(hipStreamSynchronize(st));
-		SRF_HIP(hipMemcpy(hs, timing, sizeof(hs), hipMemcpyDeviceToHost));
-		SRF_HIP(hipMemset(timing, 0, sizeof(hs)));
-		for (int i = 0; i < 1024; ++i) for (int k = 0; k < 11; ++k) h[k] += hs[i * 16 + k];
-		for (int i = 0; i < 1024; ++i) h[11] = hs[i * 16 + 11] > h[11] ? hs[i * 16 + 11] : h[11];
-		const double nw = (double)div_up(n_rays, rays_per_wave);
-		fprintf(stderr, "count march wavefront lifetime: %.0f cycles = %.1f us mean, %.1f us max\n", (double)h[9] / nw, (double)h[10] / nw / 100.0, (double)h[11] / 100.0);
-		fprintf(stderr, "count march lifetime histogram (100 us buckets):");
-		for (int k = 0; k < 48; ++k) fprintf(stderr, " %llu", hs[1024 * 16 + k]);
-		fprintf(stderr, "\ncount march probe-round histogram (buckets of 64):");
-		for (int k = 0; k < 48; ++k) fprintf(stderr, " %llu", hs[1024 * 16 + 48 + k]);
-		fprintf(stderr, "\ncount march step-round histogram (buckets of 64):");
-		for (int k = 0; k < 48; ++k) fprintf(stderr, " %llu", hs[1024 * 16 + 96 + k]);
-		fprintf(stderr, "\n");
-		{ const unsigned long long* q = hs + 1024 * 16 + 144; if (q[0]) fprintf(stderr, "count march slow wavefronts: %llu, step rounds %.0f (%.1f lanes, %.0f cycles each), probe rounds %.0f (%.1f lanes, %.0f cycles each)\n",
-			q[0], (double)q[1] / q[0], (double)q[3] / (q[1] ? q[1] : 1), (double)q[5] / (q[1] ? q[1] : 1), (double)q[2] / q[0], (double)q[4] / (q[2] ? q[2] : 1), (double)q[6] / (q[2] ? q[2] : 1)); }
-		const char* name[3] = {"step", "probe", "begin"};
-		for (int k = 0; k < 3; ++k)
-			fprintf(stderr, "count march %-5s: %.0f cycles per wavefront, %.1f rounds, %.0f cycles per round, %.1f lanes per round\n", name[k],
-			        (double)h[k] / nw, (double)h[3 + k] / nw, h[3 + k] ? (double)h[k] / (double)h[3 + k] : 0.0, h[3 + k] ? (double)h[6 + k] / (double)h[3 + k] : 0.0);
-		uint32_t n_parked = 0;
-		if (probe_budget) SRF_HIP(hipMemcpy(&n_parked, ca.parked_count, 4, hipMemcpyDeviceToHost));
-		fprintf(stderr, "count march parked rays: %u (capacity %u)\n", n_parked, parked_capacity);
-	}
-#endif
+	ca.probe_budget = ca.park_lanes = ca.parked_capacity = 0; ca.parked = nullptr; ca.parked_count = nullptr;      // (the host build's rehearsal)
+	hipLaunchKernelGGL(k_ray_order, dim3(div_up(n_rays, RAY_CHUNK)), dim3(RAY_CHUNK_BINS), 0, st, s->P, ca, order);
 	SRF_LAUNCH_CHECK();
-	if (probe_budget) {
-		const uint32_t wide_blocks = parked_capacity < 4096u ? parked_capacity : 4096u;
-		if (s->P.sphere[3] > 0.f) hipLaunchKernelGGL(k_train_count_wide<true>, dim3(wide_blocks), dim3(128), 0, st, s->P, ca);
-		else hipLaunchKernelGGL(k_train_count_wide<false>, dim3(wide_blocks), dim3(128), 0, st, s->P, ca);
-		SRF_LAUNCH_CHECK();
-	}
+	// Lanes a ray begins with: as many as keep the batch at 2^18 lanes at most, four wavefronts a SIMD (lanes at most -> time of the call:
+	// 9000 rays of the five-cascade scene 2^16: 281, 2^17: 245, 2^18: 233, 2^19: 255, 2^20: 327 us; 80 k rays 2^17: 527, 2^18: 382, 2^19: 382 us).
+	// Beyond that a lookup ahead of its time costs another ray's.
+	uint32_t team = 1;
+	while (team < 64u && (uint64_t)n_rays * team * 2u <= 262144u) team *= 2u;
+	if (s->count_team) team = s->count_team;
+	const uint32_t count_waves = div_up(n_rays, 64u / team);
+	// How far stepping lanes may be outnumbered by waiting ones: where wavefronts are many, a stepping round is cheap and worth
+	// filling the probes for (2^20 rays: ratio 4: 1266, 8: 1222, 12: 1194, 16: 1174, 32: 1217 us a call); with a few wavefronts a SIMD the
+	// lanes that wait are what the batch waits for (2^18 rays 8: 560, 16: 637 us; 80 k rays 8: 381, 32: 468 us).
+	const uint32_t probe_ratio = count_waves >= 8192u ? 16u : 8u;
+	if (s->P.sphere[3] > 0.f) hipLaunchKernelGGL(k_train_count<true>, dim3(count_waves), dim3(64), 0, st, s->P, ca, team, probe_ratio, (const uint32_t*)order);
+	else hipLaunchKernelGGL(k_train_count<false>, dim3(count_waves), dim3(64), 0, st, s->P, ca, team, probe_ratio, (const uint32_t*)order);
+	SRF_LAUNCH_CHECK();
 	const uint32_t n_tiles = div_up(n_rays, OFFSET_TILE);
 	TrainOffsetScratch os;
 	os.tile_counts = (uint32_t*)scan; os.tile_kept = os.tile_counts + n_tiles; os.tile_entries = os.tile_kept + n_tiles; os.entry = os.tile_entries + n_tiles;
