@@ -45,9 +45,9 @@ __global__ void __launch_bounds__(128) k_volume_rendering(Params P, srf_render_a
 // Single-launch compositing (phases in srf_composite_fused.h)
 // ------------------------------------------------------------------------------------
 // bytes of device scratch the chain needs for n_rays rays whose groups are cut into at most max_parts items each, and where
-// its parts lie (save_records: with room for a copy of the listed groups' ray records, see k_slow_groups)
-struct ChainLayout { size_t off_seg, off_prefix, off_misc, off_words, off_cuts, off_sums, off_items, off_list, off_side, off_saved, bytes; };
-SRF_HD constexpr ChainLayout chain_layout(uint32_t n_rays, uint32_t max_parts, bool save_records) {
+// its parts lie
+struct ChainLayout { size_t off_seg, off_prefix, off_misc, off_words, off_cuts, off_sums, off_items, off_list, off_side, bytes; };
+SRF_HD constexpr ChainLayout chain_layout(uint32_t n_rays, uint32_t max_parts) {
 	const size_t n_groups = ((size_t)n_rays + fused::RAYS - 1) / fused::RAYS;
 	const size_t n_items = (size_t)max_parts * n_groups;
 	ChainLayout L = {};
@@ -60,12 +60,11 @@ SRF_HD constexpr ChainLayout chain_layout(uint32_t n_rays, uint32_t max_parts, b
 	L.off_items = (L.off_sums + (n_groups / PREPARE_WAVES + 1) * 4 + 255) / 256 * 256;
 	L.off_list = (L.off_items + n_items * 8 + 255) / 256 * 256;
 	L.off_side = (L.off_list + n_groups * 4 + 255) / 256 * 256;
-	L.off_saved = (L.off_side + n_groups * fused::RAYS * 4 + 255) / 256 * 256;
-	L.bytes = L.off_saved + (save_records ? n_groups * fused::RAYS * 8 : 0);
+	L.bytes = L.off_side + n_groups * fused::RAYS * 4;
 	return L;
 }
-static ChainScratch chain_scratch_at(void* base, uint32_t n_rays, uint32_t max_parts, bool save_records, uint32_t* host_error, uint32_t spin_limit) {
-	const ChainLayout L = chain_layout(n_rays, max_parts, save_records);
+static ChainScratch chain_scratch_at(void* base, uint32_t n_rays, uint32_t max_parts, uint32_t* host_error, uint32_t spin_limit) {
+	const ChainLayout L = chain_layout(n_rays, max_parts);
 	ChainScratch S;
 	S.item_status = (unsigned long long*)base;
 	S.seg_status = (unsigned long long*)((char*)base + L.off_seg);
@@ -80,30 +79,30 @@ static ChainScratch chain_scratch_at(void* base, uint32_t n_rays, uint32_t max_p
 	S.items = (U2*)((char*)base + L.off_items);
 	S.slow_items = (uint32_t*)((char*)base + L.off_list);
 	S.side = (uint32_t*)((char*)base + L.off_side);
-	S.saved_records = save_records ? (U2*)((char*)base + L.off_saved) : nullptr;
 	S.host_error = host_error;
 	S.spin_limit = spin_limit;
 	S.max_parts = max_parts;
 	return S;
 }
-// Items a group may be cut into: any number where the scratch is allocated to fit; the scratch that is part of the library's
-// image (see g_noalloc_scratch) has room for eight, and groups that need more take the path of the listed ones there.
-constexpr uint32_t STREAM_MAX_PARTS = fused::MAX_PARTS;
+// A ray of more samples than this sends its group to k_long_rays: a streaming item lasts as long as its longest ray (one lane walks
+// it, some 400 cycles a sample), while there a ray has a wavefront to itself.
+constexpr uint32_t LONG_RAY = 256;
+// Items a group may be cut into: what 64 rays of that length need where the scratch is allocated to fit; the scratch that is part of
+// the library's image (see g_noalloc_scratch) has room for eight, and groups that need more take the path of the listed ones there.
+constexpr uint32_t STREAM_MAX_PARTS = (fused::RAYS * LONG_RAY + fused::GAP_SLACK) / (fused::StreamGeometry::WIN - LONG_RAY) + 1;
 constexpr uint32_t NOALLOC_MAX_PARTS = 8;
 
 // Ordering point between the phases of a group (see srf_composite_fused.h): a workgroup barrier.
 __device__ __forceinline__ void group_sync() { __syncthreads(); }
 
 // ---- groups that do not fit the streaming path ------------------------------------------------
-// The streaming kernel takes groups whose rays are laid out back to back and whose samples fit one of its windows.  The
-// others (arbitrary caller-supplied offsets; more samples than one window) are rare and are kept out of its code:
+// The streaming kernel takes groups whose rays are laid out back to back and of moderate length.  The others (arbitrary
+// caller-supplied offsets; a ray longer than LONG_RAY samples; more items than there is room for) are listed and kept out of its code:
 //   k_chain_prepare      plans every group and notes how many items it makes
 //   k_chain_items        numbers the items in ray order, clears their words of the chain and lists those of groups that the streaming path does not take
-//   k_slow_groups (fwd)  forward pass of the listed groups; leaves the number of samples every one of their rays consumes
+//   k_long_rays (fwd)    how many samples every ray of the listed groups consumes
 //   k_composite_stream   for a listed group only chains those counts to its neighbours' and leaves the rays' compacted offsets
-//   k_slow_groups (bwd)  forward pass again, then commit and gradients at those offsets
-// Rays not laid out back to back are composited one lane per ray; groups with a ray longer than a window run the window
-// phases over all windows.
+//   k_long_rays (bwd)    colours, loss, commit and gradients at those offsets
 
 // Records of one group into a plan, by the 64 lanes of one wave: what fused::plan_lane and fused::plan_finish_lane
 // compute lane by lane through LDS, with the wave's own reductions instead (64 lanes adding to one LDS word take turns).
@@ -151,6 +150,7 @@ __device__ __forceinline__ U2 load_record(uint32_t g, uint32_t lane, const fused
 __device__ __forceinline__ uint64_t plan_cuts_wave(uint32_t lane, const fused::Plan& pl, uint32_t win, uint32_t max_parts) {
 	using namespace fused;
 	if (pl.misc[M_CONTIG] == 0) return 0ull;
+	if (wave_max_fast(pl.rn[lane]) > LONG_RAY) return 0ull;
 	if (pl.misc[M_TOTAL] <= win) return 1ull;
 	const uint32_t start = pl.rbase[lane], end = pl.rbase[lane + 1];      // rbase[RAYS]: the group's end
 	uint64_t cuts = 1ull;
@@ -160,7 +160,7 @@ __device__ __forceinline__ uint64_t plan_cuts_wave(uint32_t lane, const fused::P
 		const uint64_t beyond = __ballot(end - lo_base > win) & ~((1ull << lo) - 1ull);
 		if (beyond == 0ull) return cuts;
 		const uint32_t r = (uint32_t)__builtin_ctzll(beyond);
-		if (r == lo) return 0ull;                      // ray lo alone does not fit
+		if (r == lo) return 0ull;                      // ray lo and the gap behind it do not fit
 		lo = r;
 		cuts |= 1ull << lo;
 		if (++parts > max_parts) return 0ull;
@@ -234,121 +234,159 @@ __global__ void __launch_bounds__(ITEMS_THREADS) k_chain_items(uint32_t n_rays_m
 	if (tid == 0 && g_first + ITEMS_THREADS >= n_groups) *S.n_items = all;     // the workgroup with the last group
 }
 
-struct SlowShared {
-	fused::Window<fused::WideGeometry> w;
-	fused::RayLds rl;
-	fused::Plan plan;       // the group
-	fused::Plan part;       // the rays of it that are under way
-};
+// ---- one ray a wavefront -----------------------------------------------------------------------
+// A ray's samples 64 at a time, one per lane: loads, alpha and gradients are the lanes' own, and the reference's loop (ray_marcher.cu:
+// 63-79, :171-182) runs along the lanes, each taking the value of the lane below it with a lane shift (DPP) inside the multiplication or
+// addition itself: after k of the 63 rounds lanes 0 .. k hold what the loop has after k samples, in the loop's own order of
+// operations.  Four such chains (the transmittance of one block, the colour sums of the block before it) go round together, so
+// that an instruction never waits for the lane shift of the one before it: 16 cycles a sample.
+// A walk of the ray costs nothing but its own samples, so the 4096 rays of a thousand samples of a full grid's batch take WALKFWD us
+// forward and WALKBWD us backward, where a workgroup that took such rays window by window, one lane a ray, took 6.3 and 13.4 ms.
+#define SRF_DPP_BELOW "wave_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+// x of lane k <- x of lane k-1 op y of lane k, for k = 1 .. 63 in turn (lane 0 keeps its value)
+__device__ __forceinline__ void lane_chain_mul(float& T, float F) {
+	asm("s_nop 1\n\t.rept 63\n\tv_mul_f32_dpp %0, %0, %1 " SRF_DPP_BELOW "s_nop 1\n\t.endr" : "+v"(T) : "v"(F));
+}
+__device__ __forceinline__ void lane_chains(float& T, float F, float& r, float pr, float& g, float pg, float& b, float pb) {
+	asm("s_nop 1\n\t.rept 63\n\t"
+	    "v_mul_f32_dpp %0, %0, %4 " SRF_DPP_BELOW
+	    "v_add_f32_dpp %1, %1, %5 " SRF_DPP_BELOW
+	    "v_add_f32_dpp %2, %2, %6 " SRF_DPP_BELOW
+	    "v_add_f32_dpp %3, %3, %7 " SRF_DPP_BELOW
+	    ".endr\n\ts_nop 1" : "+v"(T), "+v"(r), "+v"(g), "+v"(b) : "v"(F), "v"(pr), "v"(pg), "v"(pb));
+}
+__device__ __forceinline__ float lane_below_f32(float v) { return srf_u2f(lane_below_u32(srf_f2u(v))); }
+__device__ __forceinline__ float lane_f32(float v, uint32_t uniform_lane) { return srf_u2f(lane_value_u32(srf_f2u(v), uniform_lane)); }
 
-// Where a listed group whose rays lie back to back is cut into parts: like plan_cuts_wave, but a ray longer than a window
-// is a part of its own.  A part's rays go through the windows together and one after another part's, so that a group of long
-// rays does not walk them one behind the other; the parts of a group are dealt to `slots` units of work, which different
-// workgroups take.
-__device__ __forceinline__ uint64_t slow_cuts_wave(uint32_t lane, const fused::Plan& pl, uint32_t win) {
-	using namespace fused;
-	const uint32_t start = pl.rbase[lane], end = pl.rbase[lane + 1];
-	uint64_t cuts = 1ull;
-	uint32_t lo = 0;
-	for (;;) {
-		const uint32_t lo_base = lane_value_u32(start, lo);
-		const uint64_t beyond = __ballot(end - lo_base > win) & ~((1ull << lo) - 1ull);
-		if (beyond == 0ull) return cuts;
-		uint32_t r = (uint32_t)__builtin_ctzll(beyond);
-		if (r == lo) ++r;                              // ray lo alone is longer than a window
-		if (r >= RAYS) return cuts;
-		lo = r;
-		cuts |= 1ull << lo;
-	}
+// one sample of a ray, as its lane holds it
+template <bool HALF_IN>
+struct WalkSample { uint32_t raw[HALF_IN ? 2 : 4]; float dt; };
+template <bool HALF_IN>
+__device__ __forceinline__ void walk_load(const fused::Args& A, uint32_t base, uint32_t k, uint32_t n, WalkSample<HALF_IN>& s) {
+	if (k >= n) return;
+	const size_t at = (size_t)base + k;
+	if constexpr (HALF_IN) { const U2 p = *(const U2*)((const uint32_t*)A.net + at * 2); s.raw[0] = p.x; s.raw[1] = p.y; }
+	else { const U4 p = *(const U4*)((const uint32_t*)A.net + at * 4); s.raw[0] = p.x; s.raw[1] = p.y; s.raw[2] = p.z; s.raw[3] = p.w; }
+	s.dt = A.dt_arr[at * A.K.dt_stride];
 }
 
-constexpr uint32_t SLOW_PART_SLOTS = 16;      // workgroups that share a listed group (see k_slow_groups)
-constexpr uint32_t SLOW_WORKGROUPS = 2048;
+// The number of samples the loop consumes.
+template <bool HALF_IN>
+__device__ __forceinline__ uint32_t walk_count(uint32_t lane, const fused::Args& A, uint32_t base, uint32_t n) {
+	WalkSample<HALF_IN> next;
+	walk_load<HALF_IN>(A, base, lane, n, next);
+	float T_in = 1.f;
+	for (uint32_t k0 = 0; k0 < n; k0 += WAVE) {
+		const WalkSample<HALF_IN> s = next;
+		walk_load<HALF_IN>(A, base, k0 + WAVE + lane, n, next);
+		const bool live = k0 + lane < n;
+		float f = 1.f;
+		if (live) {
+			float v[4];
+			fused::unpack_raw<HALF_IN>(s.raw, v);
+			f = 1.f - (1.f - srf_expf(-act_density(v[3], A.K.density_act) * s.dt));
+		}
+		float T = T_in;
+		lane_chain_mul(T, lane_below_f32(f));
+		const uint64_t below = __ballot(live && T < A.K.thr);
+		if (below) return k0 + (uint32_t)__builtin_ctzll(below);
+		T_in = lane_f32(T * f, WAVE - 1u);
+	}
+	return n;
+}
+
+// The loop with colours over the first n of a ray's samples, of which all are consumed.  emit(k, s, v, alpha, {T before, colour sum}) for every
+// one of them, by the lane that holds it.  Leaves transmittance and colour in c, the same in every lane.
+template <bool HALF_IN, class Emit>
+__device__ __forceinline__ void walk_colours(uint32_t lane, const fused::Args& A, uint32_t base, uint32_t n, fused::RayCarry& c, const Emit& emit) {
+	WalkSample<HALF_IN> next, s_was{};
+	walk_load<HALF_IN>(A, base, lane, n, next);
+	float T_in = 1.f, r_in = 0.f, g_in = 0.f, b_in = 0.f;
+	float pr = 0.f, pg = 0.f, pb = 0.f;                    // weighted colours of the block before
+	float T_was = 1.f, alpha_was = 0.f;
+	for (uint32_t k0 = 0;; k0 += WAVE) {
+		const WalkSample<HALF_IN> s = next;
+		walk_load<HALF_IN>(A, base, k0 + WAVE + lane, n, next);
+		const bool live = k0 + lane < n;
+		float alpha = 0.f, f = 1.f;
+		float v[4] = {0.f, 0.f, 0.f, 0.f};
+		if (live) {
+			fused::unpack_raw<HALF_IN>(s.raw, v);
+			alpha = 1.f - srf_expf(-act_density(v[3], A.K.density_act) * s.dt);
+			f = 1.f - alpha;
+		}
+		float T = T_in, r = r_in + pr, g = g_in + pg, b = b_in + pb;      // (lane 0's; the others are overwritten)
+		lane_chains(T, lane_below_f32(f), r, pr, g, pg, b, pb);
+		if (k0 != 0) {
+			const uint32_t k = k0 - WAVE + lane;
+			if (k < n) emit(k, s_was, alpha_was, mk4(T_was, r, g, b));
+			r_in = lane_f32(r, WAVE - 1u); g_in = lane_f32(g, WAVE - 1u); b_in = lane_f32(b, WAVE - 1u);
+		}
+		if (k0 >= n) break;
+		// samples past the ray's end carry nothing: a factor of one, a colour of zero
+		const float weight = alpha * T;
+		pr = live ? weight * act_rgb(v[0], A.K.rgb_act) : 0.f; pg = live ? weight * act_rgb(v[1], A.K.rgb_act) : 0.f; pb = live ? weight * act_rgb(v[2], A.K.rgb_act) : 0.f;
+		s_was = s; T_was = T; alpha_was = alpha;
+		T_in = lane_f32(T * f, WAVE - 1u);
+	}
+	c.T = T_in; c.Cr = r_in; c.Cg = g_in; c.Cb = b_in;
+}
+
+constexpr uint32_t LONG_THREADS = 256;         // four independent wavefronts
+constexpr uint32_t LONG_WORKGROUPS = 2048;
 
 template <bool HALF_IN, bool HALF_OUT, bool BACKWARD>
-__global__ void __launch_bounds__(fused::WideGeometry::THREADS) k_slow_groups(fused::Args A, const uint32_t* __restrict__ n_rays_counter, const float* __restrict__ mean_density_ptr, ChainScratch S, uint32_t slots) {
+__global__ void __launch_bounds__(LONG_THREADS) k_long_rays(fused::Args A, const uint32_t* __restrict__ n_rays_counter, const float* __restrict__ mean_density_ptr, ChainScratch S) {
 	using namespace fused;
-	using G = WideGeometry;
-	__shared__ SlowShared sh;
-	const uint32_t tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
-	const uint32_t n_listed = *S.slow_count;
-	// a unit of work: the parts of one listed group whose number is `slot` modulo `slots`
-	const uint64_t n_units = (uint64_t)n_listed * slots;
-	if (blockIdx.x >= n_units) return;
+	const uint32_t lane = threadIdx.x % WAVE;
+	// a unit of work: one ray of a listed group
+	const uint64_t n_units = (uint64_t)*S.slow_count * RAYS;
+	uint64_t unit = (uint64_t)blockIdx.x * (LONG_THREADS / WAVE) + threadIdx.x / WAVE;
+	if (unit >= n_units) return;
 	const uint32_t counter_now = *n_rays_counter;
 	A.mean_density = mean_density_ptr ? *mean_density_ptr : 0.f;
 	A.n_active = counter_now < A.K.n_rays ? counter_now : A.K.n_rays;
-	if (!BACKWARD) A.rgb_ray_out = nullptr;      // written once, by the second forward pass
-	for (uint64_t unit = blockIdx.x; unit < n_units; unit += gridDim.x) {
-		const uint32_t k = (uint32_t)(unit / slots), slot = (uint32_t)(unit % slots);
-		const uint32_t g = S.items[S.slow_items[k]].x;
-		const uint32_t ray0 = g * RAYS;
-		if (wave == 0) {
-			// The commit of the backward launch overwrites a ray's record, and the workgroups that share a group do not wait for
-			// one another: they plan from the copy that the forward launch left.
-			U2 rec;
-			if (BACKWARD && S.saved_records) rec = S.saved_records[(size_t)ray0 + lane];
-			else {
-				rec = load_record(g, lane, A);
-				if (S.saved_records && slot == 0) S.saved_records[(size_t)ray0 + lane] = rec;
-			}
-			plan_from_records(lane, g, rec, A, sh.plan);
+	for (; unit < n_units; unit += (uint64_t)gridDim.x * (LONG_THREADS / WAVE)) {
+		const uint32_t i = SRF_UNIFORM_U32(S.items[S.slow_items[unit / RAYS]].x * RAYS + (uint32_t)(unit % RAYS));
+		if (i >= A.n_active) continue;
+		const U2 rec = *(const U2*)(A.ray_coord_indices + 2 * (size_t)i);
+		const uint32_t numsteps = SRF_UNIFORM_U32(rec.x), base = SRF_UNIFORM_U32(rec.y);
+		const uint32_t n_fwd = walk_count<HALF_IN>(lane, A, base, numsteps);
+		if (!BACKWARD) {
+			if (lane == 0) S.side[i] = n_fwd;
+			continue;
 		}
-		group_sync();
-		if (sh.plan.misc[M_CONTIG] != 0) {
-			uint64_t cuts = slow_cuts_wave(lane, sh.plan, G::WIN);      // (the same in every wave)
-			for (uint32_t part_number = 0; cuts != 0ull; ++part_number) {
-				const uint32_t lo = (uint32_t)__builtin_ctzll(cuts);
-				cuts &= cuts - 1ull;
-				const uint32_t hi = cuts ? (uint32_t)__builtin_ctzll(cuts) : RAYS;
-				if (part_number % slots != slot) continue;
-				const Plan& pl = sh.part;
-				if (wave == 0) plan_part_lane(lane, sh.plan, lo, hi, g, sh.part);
-				group_sync();
-				const bool live = wave == 0 && ray0 + lane < A.n_active && lane >= lo && lane < hi;
-				const uint32_t n_win = (pl.misc[M_TOTAL] + G::WIN - 1) / G::WIN;
-				SlotState<G, HALF_IN> st;
-				RayCarry c;
-				Float4 target = mk4(0.f, 0.f, 0.f, 0.f);
-				if (live) target = *(const Float4*)(A.rays_rgba + 4 * (size_t)(ray0 + lane));
-				if (wave == 0) reset_carry(lane, pl, c);
-				for (uint32_t win = 0; win < n_win; ++win) {
-					phase_a<G, HALF_IN>(tid, win, A, sh.w, pl, st);
-					group_sync();
-					if (wave == 0) chain<G>(lane, win, A, sh.w, sh.rl, pl, c);
-					group_sync();
-				}
-				if (wave == 0) finish_ray(lane, ray0, A, sh.rl, c, target, lo, hi);
-				if (!BACKWARD) {
-					if (live) S.side[ray0 + lane] = sh.rl.rnf[lane];
-				} else {
-					if (wave == 0) commit_ray(lane, ray0, live ? S.side[ray0 + lane] : 0u, A, sh.rl, pl, lo, hi);
-					group_sync();
-					if (wave == 0) reset_carry(lane, pl, c);
-					for (uint32_t win = 0; win < n_win; ++win) {
-						phase_a<G, HALF_IN>(tid, win, A, sh.w, pl, st);
-						group_sync();
-						if (wave == 0) chain<G>(lane, win, A, sh.w, sh.rl, pl, c);
-						group_sync();
-						phase_c<G, HALF_IN, HALF_OUT>(tid, win, A, sh.w, sh.rl, pl, st);
-						group_sync();
-					}
-				}
-				group_sync();
-			}
-		} else if (wave == 0 && slot == 0) {
-			const bool live = ray0 + lane < A.n_active;
-			uint32_t n = 0;
-			FwdRay fw;
-			loss_forward_body<HALF_IN>(ray0 + lane, A.K, A.rays_rgba, A.n_active, A.ray_coord_indices, A.dt_arr, A.net, &fw, &n, A.rgb_ray_out);
-			if (!BACKWARD) {
-				if (live) S.side[ray0 + lane] = n;
-			} else if (live) {
-				loss_backward_body<HALF_IN, HALF_OUT>(ray0 + lane, A.K, A.n_active, A.ray_coord_indices, A.dt_arr, A.coords, A.compacted_coords, A.net, A.dloss, A.loss_output,
-				                                      A.mean_density, fw, n, S.side[ray0 + lane], nullptr);
-			}
+		RayCarry c;
+		walk_colours<HALF_IN>(lane, A, base, n_fwd, c, [](uint32_t, const WalkSample<HALF_IN>&, float, Float4) {});
+		// finish_ray and commit_ray for one ray (ray_marcher.cu:81-133)
+		float target[3], bg[3];
+		target_and_background(A.K, *(const Float4*)(A.rays_rgba + 4 * (size_t)i), target, bg);
+		if (n_fwd == numsteps) { c.Cr += c.T * bg[0]; c.Cg += c.T * bg[1]; c.Cb += c.T * bg[2]; }
+		float lo[3];
+		Float4 og = mk4(0.f, 0.f, 0.f, 0.f);
+		loss_channel(A.K.loss_type, target[0], c.Cr, &lo[0], &og.x);
+		loss_channel(A.K.loss_type, target[1], c.Cg, &lo[1], &og.y);
+		loss_channel(A.K.loss_type, target[2], c.Cb, &lo[2], &og.z);
+		const uint32_t cbase = S.side[i];
+		const uint32_t room = A.K.n_max_compacted - (A.K.n_max_compacted < cbase ? A.K.n_max_compacted : cbase);
+		const uint32_t n = room < n_fwd ? room : n_fwd;
+		if (lane == 0) {
+			if (A.rgb_ray_out) { A.rgb_ray_out[3 * (size_t)i] = c.Cr; A.rgb_ray_out[3 * (size_t)i + 1] = c.Cg; A.rgb_ray_out[3 * (size_t)i + 2] = c.Cb; }
+			A.ray_coord_indices[2 * (size_t)i] = n;
+			A.ray_coord_indices[2 * (size_t)i + 1] = cbase;
+			if (n != 0 && A.loss_output) A.loss_output[i] = (((lo[0] + lo[1]) + lo[2]) / 3.0f) / (float)A.K.n_rays;
 		}
-		group_sync();
+		const Float4 oc = mk4(c.Cr, c.Cg, c.Cb, 0.f);
+		walk_colours<HALF_IN>(lane, A, base, n, c, [&](uint32_t k, const WalkSample<HALF_IN>& s, float alpha, Float4 after) {
+			float v[4];
+			unpack_raw<HALF_IN>(s.raw, v);
+			sample_gradient<HALF_OUT, false>(A, v, s.dt, alpha, after, og, oc, (size_t)cbase + k);
+		});
+		if (A.compacted_coords) {
+			const float* src = A.coords + 7 * (size_t)base;
+			float* dst = A.compacted_coords + 7 * (size_t)cbase;
+			for (uint32_t k = lane; k < 7u * n; k += WAVE) dst[k] = src[k];
+		}
 	}
 }
 
@@ -761,13 +799,14 @@ static int launch_stream(const srf_loss_args* a, const LossConst& K, ChainScratc
 #undef SRF_RESIDENT_IO
 #undef SRF_RESIDENT
 	if (rc != SRF_OK) return rc;
-	const dim3 grid(n_groups < resident ? n_groups : resident), block(STREAM_THREADS), slow_block(fused::WideGeometry::THREADS), slow_grid(n_groups < SLOW_WORKGROUPS ? n_groups : SLOW_WORKGROUPS);   // listed groups are few as a rule
-	const uint32_t slow_slots = S.saved_records ? SLOW_PART_SLOTS : 1u;       // without the copy of their records a group is one workgroup's
+	const dim3 grid(n_groups < resident ? n_groups : resident), block(STREAM_THREADS), long_block(LONG_THREADS);
+	const uint32_t long_groups = div_up(n_groups * fused::RAYS, LONG_THREADS / WAVE);
+	const dim3 long_grid(long_groups < LONG_WORKGROUPS ? long_groups : LONG_WORKGROUPS);   // listed groups are few as a rule
 	hipLaunchKernelGGL(k_chain_prepare, dim3(div_up(n_groups, PREPARE_WAVES)), dim3(PREPARE_WAVES * WAVE), 0, st, A, n_rays_counter, S, (const uint32_t*)n_compacted_coords_counter);
 	hipLaunchKernelGGL(k_chain_items, dim3(div_up(n_groups, ITEMS_THREADS)), dim3(ITEMS_THREADS), 0, st, a->n_rays, n_rays_counter, S);
 	SRF_LAUNCH_CHECK();
-	if (hin) hipLaunchKernelGGL((k_slow_groups<true, false, false>), slow_grid, slow_block, 0, st, A, n_rays_counter, density_grid_mean, S, slow_slots);
-	else     hipLaunchKernelGGL((k_slow_groups<false, false, false>), slow_grid, slow_block, 0, st, A, n_rays_counter, density_grid_mean, S, slow_slots);
+	if (hin) hipLaunchKernelGGL((k_long_rays<true, false, false>), long_grid, long_block, 0, st, A, n_rays_counter, density_grid_mean, S);
+	else     hipLaunchKernelGGL((k_long_rays<false, false, false>), long_grid, long_block, 0, st, A, n_rays_counter, density_grid_mean, S);
 	SRF_LAUNCH_CHECK();
 #define SRF_STREAM(HI, HO, PL) hipLaunchKernelGGL((k_composite_stream<HI, HO, PL>), grid, block, 0, st, A, n_rays_counter, density_grid_mean, S, n_compacted_coords_counter)
 #define SRF_STREAM_IO(PL) do { if (hin && hout) SRF_STREAM(true, true, PL); else if (hin) SRF_STREAM(true, false, PL); else if (hout) SRF_STREAM(false, true, PL); else SRF_STREAM(false, false, PL); } while (0)
@@ -775,9 +814,9 @@ static int launch_stream(const srf_loss_args* a, const LossConst& K, ChainScratc
 #undef SRF_STREAM_IO
 #undef SRF_STREAM
 	SRF_LAUNCH_CHECK();
-#define SRF_SLOW_BWD(HI, HO) hipLaunchKernelGGL((k_slow_groups<HI, HO, true>), slow_grid, slow_block, 0, st, A, n_rays_counter, density_grid_mean, S, slow_slots)
-	if (hin && hout) SRF_SLOW_BWD(true, true); else if (hin) SRF_SLOW_BWD(true, false); else if (hout) SRF_SLOW_BWD(false, true); else SRF_SLOW_BWD(false, false);
-#undef SRF_SLOW_BWD
+#define SRF_LONG_BWD(HI, HO) hipLaunchKernelGGL((k_long_rays<HI, HO, true>), long_grid, long_block, 0, st, A, n_rays_counter, density_grid_mean, S)
+	if (hin && hout) SRF_LONG_BWD(true, true); else if (hin) SRF_LONG_BWD(true, false); else if (hout) SRF_LONG_BWD(false, true); else SRF_LONG_BWD(false, false);
+#undef SRF_LONG_BWD
 	SRF_LAUNCH_CHECK();
 #ifdef SRF_KERNEL_TIMING
 	{
@@ -911,7 +950,7 @@ static int loss_call_prepare(srf_marcher* m, const srf_loss_args* a, const float
 // The chain's scratch for srf_marcher_volume_rendering_with_loss_and_gradient_noalloc: part of the library's image on every
 // device, found once per device with hipGetSymbolAddress (the array's name means nothing to host code).
 constexpr uint32_t NOALLOC_MAX_RAYS = SRF_NOALLOC_MAX_RAYS;
-constexpr size_t NOALLOC_BYTES = chain_layout(NOALLOC_MAX_RAYS, NOALLOC_MAX_PARTS, false).bytes;
+constexpr size_t NOALLOC_BYTES = chain_layout(NOALLOC_MAX_RAYS, NOALLOC_MAX_PARTS).bytes;
 static __device__ __align__(256) unsigned char g_noalloc_scratch[NOALLOC_BYTES];
 constexpr int NOALLOC_MAX_DEVICES = 64;
 static void* g_noalloc_ptr[NOALLOC_MAX_DEVICES];      // per device: where g_noalloc_scratch lies in its memory
@@ -1030,10 +1069,10 @@ int srf_marcher_volume_rendering_with_loss_and_gradient(srf_marcher_t* m, const 
 		                    compacted_coords, n_compacted_coords_counter, network_output, dloss_doutput, loss_output, density_grid_mean, rgb_ray_out, st);
 	}
 	if (fusable && level == 0) {
-		rc = m->ws.reserve(chain_layout(a->n_rays, STREAM_MAX_PARTS, true).bytes);
+		rc = m->ws.reserve(chain_layout(a->n_rays, STREAM_MAX_PARTS).bytes);
 		if (rc != SRF_OK) return rc;
-		m->chain_error_dev = chain_scratch_at(m->ws.ptr, a->n_rays, STREAM_MAX_PARTS, true, nullptr, 0).error;
-		return launch_stream(a, K, chain_scratch_at(m->ws.ptr, a->n_rays, STREAM_MAX_PARTS, true, m->host_error_dev, m->lookback_spin_limit), rays_rgba, n_rays_counter, ray_coord_indices, dt, coords,
+		m->chain_error_dev = chain_scratch_at(m->ws.ptr, a->n_rays, STREAM_MAX_PARTS, nullptr, 0).error;
+		return launch_stream(a, K, chain_scratch_at(m->ws.ptr, a->n_rays, STREAM_MAX_PARTS, m->host_error_dev, m->lookback_spin_limit), rays_rgba, n_rays_counter, ray_coord_indices, dt, coords,
 		                     compacted_coords, n_compacted_coords_counter, network_output, dloss_doutput, loss_output, density_grid_mean, rgb_ray_out, st);
 	}
 
@@ -1090,8 +1129,8 @@ int srf_marcher_volume_rendering_with_loss_and_gradient_noalloc(srf_marcher_t* m
 	void* scratch = nullptr;
 	rc = noalloc_scratch(&scratch);
 	if (rc != SRF_OK) return rc;
-	m->chain_error_dev = chain_scratch_at(scratch, a->n_rays, NOALLOC_MAX_PARTS, false, nullptr, 0).error;
-	return launch_stream(a, K, chain_scratch_at(scratch, a->n_rays, NOALLOC_MAX_PARTS, false, m->host_error_dev, m->lookback_spin_limit), rays_rgba, n_rays_counter, ray_coord_indices, dt, coords,
+	m->chain_error_dev = chain_scratch_at(scratch, a->n_rays, NOALLOC_MAX_PARTS, nullptr, 0).error;
+	return launch_stream(a, K, chain_scratch_at(scratch, a->n_rays, NOALLOC_MAX_PARTS, m->host_error_dev, m->lookback_spin_limit), rays_rgba, n_rays_counter, ray_coord_indices, dt, coords,
 	                     compacted_coords, n_compacted_coords_counter, network_output, dloss_doutput, loss_output, density_grid_mean, rgb_ray_out, (hipStream_t)stream);
 }
 

@@ -64,7 +64,7 @@ struct Geometry {
 	static constexpr uint32_t WIN = THREADS_ * SLOTS_;   // samples per window
 	static constexpr bool FENCE_SLOTS = FENCE_SLOTS_;
 };
-// a whole workgroup of four waves on the samples, windows of 1792: the kernel for groups of any length
+// a whole workgroup of four waves on the samples, windows of 1792: groups of any length (the host build's rehearsal of them)
 using WideGeometry = Geometry<256, 7, true>;
 // six waves on the samples (two more walk the rays and plan meanwhile), windows of 1920: the streaming kernel
 using StreamGeometry = Geometry<384, 5, false>;
@@ -560,13 +560,49 @@ SRF_HD void commit_loss(uint32_t lane, uint32_t ray0, const Args& A, const RayLd
 	if (rl.out[lane].s_end != pl.rbase[lane] && A.loss_output) A.loss_output[i] = rl.loss[lane];
 }
 
+// the gradient of one kept sample (ray_marcher.cu:171-201), stored as record o: v what the network gave, after {T before the sample,
+// colour sum including it}, og.xyz d loss / d colour, oc.xyz the composited colour
+template <bool HALF_OUT, bool PLAIN>
+SRF_HD void sample_gradient(const Args& A, const float v[4], float dt, float alpha, Float4 after, Float4 og, Float4 oc, size_t o) {
+	const int rgb_act = PLAIN ? (int)SRF_ACT_NONE : A.K.rgb_act, density_act = PLAIN ? (int)SRF_ACT_NONE : A.K.density_act;
+	const float l2_reg = rgb_act == SRF_ACT_EXPONENTIAL ? 1e-4f : 0.0f;
+	const float l1_reg_density = (A.K.use_grid && (A.mean_density < A.K.min_optical_thickness)) ? 1e-4f : 0.0f;
+	const float T_before = after.x;
+	const float cr = act_rgb(v[0], rgb_act), cg = act_rgb(v[1], rgb_act), cb = act_rgb(v[2], rgb_act);
+	const float weight = alpha * T_before;
+	const float T = T_before * (1.f - alpha);                // the chain's own update (ray_marcher.cu:181)
+	const float d0 = A.K.loss_scale * ((weight * og.x) * act_rgb_derivative(v[0], rgb_act) + srf_max_zero(l2_reg * v[0]));
+	const float d1 = A.K.loss_scale * ((weight * og.y) * act_rgb_derivative(v[1], rgb_act) + srf_max_zero(l2_reg * v[1]));
+	const float d2 = A.K.loss_scale * ((weight * og.z) * act_rgb_derivative(v[2], rgb_act) + srf_max_zero(l2_reg * v[2]));
+	const float sx = oc.x - after.y, sy = oc.y - after.z, sz = oc.z - after.w;
+	const float dd = act_density_derivative(v[3], density_act);
+	const float dotv = (og.x * (T * cr - sx) + og.y * (T * cg - sy)) + og.z * (T * cb - sz);
+	const float dmlp = dd * (dt * dotv);
+	const float d3 = A.K.loss_scale * dmlp + (v[3] < 0 ? -l1_reg_density : 0.0f);
+	// One vector store per sample when the records are 4 wide (the reference's padded_output_width).  The general
+	// case goes through volatile pointers only to keep the compiler from folding both cases into scalar stores.
+	if (HALF_OUT) {
+		const uint32_t lo = (uint32_t)float_to_half_bits(d0) | ((uint32_t)float_to_half_bits(d1) << 16);
+		const uint32_t hi = (uint32_t)float_to_half_bits(d2) | ((uint32_t)float_to_half_bits(d3) << 16);
+		if (A.K.out_width == 4) {
+			U2 r; r.x = lo; r.y = hi;
+			*((U2*)A.dloss + o) = r;
+		} else {
+			volatile uint16_t* p = (volatile uint16_t*)A.dloss + o * A.K.out_width;
+			p[0] = (uint16_t)(lo & 0xffffu); p[1] = (uint16_t)(lo >> 16); p[2] = (uint16_t)(hi & 0xffffu); p[3] = (uint16_t)(hi >> 16);
+		}
+	} else if (A.K.out_width == 4) {
+		*((Float4*)A.dloss + o) = mk4(d0, d1, d2, d3);
+	} else {
+		volatile float* p = (volatile float*)A.dloss + o * A.K.out_width;
+		p[0] = d0; p[1] = d1; p[2] = d2; p[3] = d3;
+	}
+}
+
 // ---- phase C: thread <-> sample (ray_marcher.cu:171-201) ---------------------------------
 // COPY_COORDS = false: the kept samples' coordinates are moved elsewhere (coords_copy_single)
 template <class G, bool HALF_IN, bool HALF_OUT, bool PLAIN = false, bool COPY_COORDS = true>
 SRF_HD void phase_c(uint32_t tid, uint32_t win, const Args& A, const Window<G>& w, const RayLds& rl, const Plan& pl, SlotState<G, HALF_IN>& st) {
-	const int rgb_act = PLAIN ? (int)SRF_ACT_NONE : A.K.rgb_act, density_act = PLAIN ? (int)SRF_ACT_NONE : A.K.density_act;
-	const float l2_reg = rgb_act == SRF_ACT_EXPONENTIAL ? 1e-4f : 0.0f;
-	const float l1_reg_density = (A.K.use_grid && (A.mean_density < A.K.min_optical_thickness)) ? 1e-4f : 0.0f;
 	const uint32_t total = pl.misc[M_TOTAL];
 	const uint32_t in_window = total - win * G::WIN < G::WIN ? total - win * G::WIN : G::WIN;
 	const uint32_t n_slots = (in_window + G::THREADS - 1) / G::THREADS;
@@ -582,40 +618,10 @@ SRF_HD void phase_c(uint32_t tid, uint32_t win, const Args& A, const Window<G>& 
 		const Float4 og = *(const Float4*)&rl.out[r].g[0];      // g.xyz, obase
 		const Float4 oc = *(const Float4*)&rl.out[r].c[0];      // c.xyz, s_end
 		if (srel >= srf_f2u(oc.w)) continue;
-		const Float4 after = w.S[q];                             // T before the sample, colour sum including it
-		const float T_before = after.x;
 		float v[4];
 		unpack_raw<HALF_IN>(st.raw[j], v);
-		const float cr = act_rgb(v[0], rgb_act), cg = act_rgb(v[1], rgb_act), cb = act_rgb(v[2], rgb_act);
-		const float weight = st.alpha[j] * T_before;
-		const float T = T_before * (1.f - st.alpha[j]);          // the chain's own update (ray_marcher.cu:181)
-		const float d0 = A.K.loss_scale * ((weight * og.x) * act_rgb_derivative(v[0], rgb_act) + srf_max_zero(l2_reg * v[0]));
-		const float d1 = A.K.loss_scale * ((weight * og.y) * act_rgb_derivative(v[1], rgb_act) + srf_max_zero(l2_reg * v[1]));
-		const float d2 = A.K.loss_scale * ((weight * og.z) * act_rgb_derivative(v[2], rgb_act) + srf_max_zero(l2_reg * v[2]));
-		const float sx = oc.x - after.y, sy = oc.y - after.z, sz = oc.z - after.w;
-		const float dd = act_density_derivative(v[3], density_act);
-		const float dotv = (og.x * (T * cr - sx) + og.y * (T * cg - sy)) + og.z * (T * cb - sz);
-		const float dmlp = dd * (st.dt[j] * dotv);
-		const float d3 = A.K.loss_scale * dmlp + (v[3] < 0 ? -l1_reg_density : 0.0f);
 		const size_t o = (size_t)(uint32_t)(srf_f2u(og.w) + srel);
-		// One vector store per sample when the records are 4 wide (the reference's padded_output_width).  The general
-		// case goes through volatile pointers only to keep the compiler from folding both cases into scalar stores.
-		if (HALF_OUT) {
-			const uint32_t lo = (uint32_t)float_to_half_bits(d0) | ((uint32_t)float_to_half_bits(d1) << 16);
-			const uint32_t hi = (uint32_t)float_to_half_bits(d2) | ((uint32_t)float_to_half_bits(d3) << 16);
-			if (A.K.out_width == 4) {
-				U2 v; v.x = lo; v.y = hi;
-				*((U2*)A.dloss + o) = v;
-			} else {
-				volatile uint16_t* p = (volatile uint16_t*)A.dloss + o * A.K.out_width;
-				p[0] = (uint16_t)(lo & 0xffffu); p[1] = (uint16_t)(lo >> 16); p[2] = (uint16_t)(hi & 0xffffu); p[3] = (uint16_t)(hi >> 16);
-			}
-		} else if (A.K.out_width == 4) {
-			*((Float4*)A.dloss + o) = mk4(d0, d1, d2, d3);
-		} else {
-			volatile float* p = (volatile float*)A.dloss + o * A.K.out_width;
-			p[0] = d0; p[1] = d1; p[2] = d2; p[3] = d3;
-		}
+		sample_gradient<HALF_OUT, PLAIN>(A, v, st.dt[j], st.alpha[j], w.S[q], og, oc, o);
 		if (COPY_COORDS && A.compacted_coords) {
 			const size_t s = (size_t)pl.misc[M_S0] + (size_t)win * G::WIN + q;
 			float cc[7];
