@@ -44,9 +44,21 @@ __global__ void __launch_bounds__(128) k_volume_rendering(Params P, srf_render_a
 // ------------------------------------------------------------------------------------
 // Single-launch compositing (phases in srf_composite_fused.h)
 // ------------------------------------------------------------------------------------
+// A ray of more samples than this sends its group to k_long_rays: a streaming item lasts as long as its longest ray (one lane walks
+// it, some 400 cycles a sample), while there a ray has a wavefront to itself.  (64: workload 4's compositing 231 -> 374 us, since groups of
+// ordinary rays go there too; 96 to 256 make no difference to it.)
+constexpr uint32_t LONG_RAY = 128;
+// What the forward walk of a long ray leaves: the gradient of the loss, how many samples the ray consumes, its colour, its first
+// sample, and where the loop stands at the beginning of each of eight stretches {transmittance, colour sum}, which the backward walk
+// then takes side by side.  Kept for the first LONG_SAVED rays; with more, the others' stretches would have to wait anyway, and the
+// backward walk of such a ray begins from its first sample.
+constexpr uint32_t LONG_STRETCHES = 8;
+struct alignas(16) LongRay { float g[3]; uint32_t n_fwd; float c[3]; uint32_t base; uint32_t stretch, pad[3]; Float4 at[LONG_STRETCHES]; };
+constexpr uint32_t LONG_SAVED = 32768;
+
 // bytes of device scratch the chain needs for n_rays rays whose groups are cut into at most max_parts items each, and where
 // its parts lie
-struct ChainLayout { size_t off_seg, off_prefix, off_misc, off_words, off_cuts, off_sums, off_items, off_list, off_side, bytes; };
+struct ChainLayout { size_t off_seg, off_prefix, off_misc, off_words, off_cuts, off_sums, off_items, off_list, off_side, off_long, bytes; };
 SRF_HD constexpr ChainLayout chain_layout(uint32_t n_rays, uint32_t max_parts) {
 	const size_t n_groups = ((size_t)n_rays + fused::RAYS - 1) / fused::RAYS;
 	const size_t n_items = (size_t)max_parts * n_groups;
@@ -60,7 +72,8 @@ SRF_HD constexpr ChainLayout chain_layout(uint32_t n_rays, uint32_t max_parts) {
 	L.off_items = (L.off_sums + (n_groups / PREPARE_WAVES + 1) * 4 + 255) / 256 * 256;
 	L.off_list = (L.off_items + n_items * 8 + 255) / 256 * 256;
 	L.off_side = (L.off_list + n_groups * 4 + 255) / 256 * 256;
-	L.bytes = L.off_side + n_groups * fused::RAYS * 4;
+	L.off_long = (L.off_side + n_groups * fused::RAYS * 4 + 255) / 256 * 256;
+	L.bytes = L.off_long + (n_groups * fused::RAYS < LONG_SAVED ? n_groups * fused::RAYS : LONG_SAVED) * sizeof(LongRay);
 	return L;
 }
 static ChainScratch chain_scratch_at(void* base, uint32_t n_rays, uint32_t max_parts, uint32_t* host_error, uint32_t spin_limit) {
@@ -79,14 +92,12 @@ static ChainScratch chain_scratch_at(void* base, uint32_t n_rays, uint32_t max_p
 	S.items = (U2*)((char*)base + L.off_items);
 	S.slow_items = (uint32_t*)((char*)base + L.off_list);
 	S.side = (uint32_t*)((char*)base + L.off_side);
+	S.long_rays = (char*)base + L.off_long;
 	S.host_error = host_error;
 	S.spin_limit = spin_limit;
 	S.max_parts = max_parts;
 	return S;
 }
-// A ray of more samples than this sends its group to k_long_rays: a streaming item lasts as long as its longest ray (one lane walks
-// it, some 400 cycles a sample), while there a ray has a wavefront to itself.
-constexpr uint32_t LONG_RAY = 256;
 // Items a group may be cut into: what 64 rays of that length need where the scratch is allocated to fit; the scratch that is part of
 // the library's image (see g_noalloc_scratch) has room for eight, and groups that need more take the path of the listed ones there.
 constexpr uint32_t STREAM_MAX_PARTS = (fused::RAYS * LONG_RAY + fused::GAP_SLACK) / (fused::StreamGeometry::WIN - LONG_RAY) + 1;
@@ -239,14 +250,12 @@ __global__ void __launch_bounds__(ITEMS_THREADS) k_chain_items(uint32_t n_rays_m
 // 63-79, :171-182) runs along the lanes, each taking the value of the lane below it with a lane shift (DPP) inside the multiplication or
 // addition itself: after k of the 63 rounds lanes 0 .. k hold what the loop has after k samples, in the loop's own order of
 // operations.  Four such chains (the transmittance of one block, the colour sums of the block before it) go round together, so
-// that an instruction never waits for the lane shift of the one before it: 16 cycles a sample.
-// A walk of the ray costs nothing but its own samples, so the 4096 rays of a thousand samples of a full grid's batch take WALKFWD us
-// forward and WALKBWD us backward, where a workgroup that took such rays window by window, one lane a ray, took 6.3 and 13.4 ms.
+// that an instruction never waits for the lane shift of the one before it: 16 cycles a sample.  Bound by that chain's latency: the
+// forward walk notes where the loop stands eight times a ray, and backward eight wavefronts take the stretches between.  The 4096 rays of a
+// thousand samples of a full grid's batch take WALKFWD us forward and WALKBWD us backward (one wavefront a ray backward, the forward
+// loop redone: 208 us; a workgroup that took such rays window by window, one lane a ray: 6.3 and 13.4 ms).
 #define SRF_DPP_BELOW "wave_shr:1 row_mask:0xf bank_mask:0xf\n\t"
 // x of lane k <- x of lane k-1 op y of lane k, for k = 1 .. 63 in turn (lane 0 keeps its value)
-__device__ __forceinline__ void lane_chain_mul(float& T, float F) {
-	asm("s_nop 1\n\t.rept 63\n\tv_mul_f32_dpp %0, %0, %1 " SRF_DPP_BELOW "s_nop 1\n\t.endr" : "+v"(T) : "v"(F));
-}
 __device__ __forceinline__ void lane_chains(float& T, float F, float& r, float pr, float& g, float pg, float& b, float pb) {
 	asm("s_nop 1\n\t.rept 63\n\t"
 	    "v_mul_f32_dpp %0, %0, %4 " SRF_DPP_BELOW
@@ -270,44 +279,19 @@ __device__ __forceinline__ void walk_load(const fused::Args& A, uint32_t base, u
 	s.dt = A.dt_arr[at * A.K.dt_stride];
 }
 
-// The number of samples the loop consumes.
-template <bool HALF_IN>
-__device__ __forceinline__ uint32_t walk_count(uint32_t lane, const fused::Args& A, uint32_t base, uint32_t n) {
-	WalkSample<HALF_IN> next;
-	walk_load<HALF_IN>(A, base, lane, n, next);
-	float T_in = 1.f;
-	for (uint32_t k0 = 0; k0 < n; k0 += WAVE) {
-		const WalkSample<HALF_IN> s = next;
-		walk_load<HALF_IN>(A, base, k0 + WAVE + lane, n, next);
-		const bool live = k0 + lane < n;
-		float f = 1.f;
-		if (live) {
-			float v[4];
-			fused::unpack_raw<HALF_IN>(s.raw, v);
-			f = 1.f - (1.f - srf_expf(-act_density(v[3], A.K.density_act) * s.dt));
-		}
-		float T = T_in;
-		lane_chain_mul(T, lane_below_f32(f));
-		const uint64_t below = __ballot(live && T < A.K.thr);
-		if (below) return k0 + (uint32_t)__builtin_ctzll(below);
-		T_in = lane_f32(T * f, WAVE - 1u);
-	}
-	return n;
-}
-
-// The loop with colours over the first n of a ray's samples, of which all are consumed.  emit(k, s, v, alpha, {T before, colour sum}) for every
-// one of them, by the lane that holds it.  Leaves transmittance and colour in c, the same in every lane.
-template <bool HALF_IN, class Emit>
-__device__ __forceinline__ void walk_colours(uint32_t lane, const fused::Args& A, uint32_t base, uint32_t n, fused::RayCarry& c, const Emit& emit) {
-	WalkSample<HALF_IN> next, s_was{};
-	walk_load<HALF_IN>(A, base, lane, n, next);
-	float T_in = 1.f, r_in = 0.f, g_in = 0.f, b_in = 0.f;
+// The loop over a ray's samples [k, n) from where `c` stands (transmittance and colour, the same in every lane), k a multiple of 64.
+// COUNT: until the reference's test ends it; returns where that is (else n).  emit(k, s, alpha, {T before, colour sum}) for every sample, by
+// the lane that holds it; at_block(k, {T, colour}) before every 64 samples.
+template <bool HALF_IN, bool COUNT, class Emit, class AtBlock>
+__device__ __forceinline__ uint32_t walk(uint32_t lane, const fused::Args& A, uint32_t base, uint32_t k, uint32_t n, fused::RayCarry& c, const Emit& emit, const AtBlock& at_block) {
+	WalkSample<HALF_IN> next{}, s_was{};
+	walk_load<HALF_IN>(A, base, k + lane, n, next);
 	float pr = 0.f, pg = 0.f, pb = 0.f;                    // weighted colours of the block before
 	float T_was = 1.f, alpha_was = 0.f;
-	for (uint32_t k0 = 0;; k0 += WAVE) {
+	for (bool first = true;; k += WAVE, first = false) {
 		const WalkSample<HALF_IN> s = next;
-		walk_load<HALF_IN>(A, base, k0 + WAVE + lane, n, next);
-		const bool live = k0 + lane < n;
+		walk_load<HALF_IN>(A, base, k + WAVE + lane, n, next);
+		const bool live = k + lane < n;
 		float alpha = 0.f, f = 1.f;
 		float v[4] = {0.f, 0.f, 0.f, 0.f};
 		if (live) {
@@ -315,77 +299,132 @@ __device__ __forceinline__ void walk_colours(uint32_t lane, const fused::Args& A
 			alpha = 1.f - srf_expf(-act_density(v[3], A.K.density_act) * s.dt);
 			f = 1.f - alpha;
 		}
-		float T = T_in, r = r_in + pr, g = g_in + pg, b = b_in + pb;      // (lane 0's; the others are overwritten)
+		float T = c.T, r = c.Cr + pr, g = c.Cg + pg, b = c.Cb + pb;      // (lane 0's; the others are overwritten)
 		lane_chains(T, lane_below_f32(f), r, pr, g, pg, b, pb);
-		if (k0 != 0) {
-			const uint32_t k = k0 - WAVE + lane;
-			if (k < n) emit(k, s_was, alpha_was, mk4(T_was, r, g, b));
-			r_in = lane_f32(r, WAVE - 1u); g_in = lane_f32(g, WAVE - 1u); b_in = lane_f32(b, WAVE - 1u);
+		if (!first) {
+			if (k - WAVE + lane < n) emit(k - WAVE + lane, s_was, alpha_was, mk4(T_was, r, g, b));
+			c.Cr = lane_f32(r, WAVE - 1u); c.Cg = lane_f32(g, WAVE - 1u); c.Cb = lane_f32(b, WAVE - 1u);
 		}
-		if (k0 >= n) break;
-		// samples past the ray's end carry nothing: a factor of one, a colour of zero
+		if (k >= n) return n;
+		at_block(k, c);
+		uint32_t end = n;
+		if (COUNT) {
+			const uint64_t below = __ballot(live && T < A.K.thr);
+			if (below) end = k + (uint32_t)__builtin_ctzll(below);
+		}
+		// samples past the end carry nothing: a factor of one, a colour of zero
+		const bool kept = k + lane < end;
 		const float weight = alpha * T;
-		pr = live ? weight * act_rgb(v[0], A.K.rgb_act) : 0.f; pg = live ? weight * act_rgb(v[1], A.K.rgb_act) : 0.f; pb = live ? weight * act_rgb(v[2], A.K.rgb_act) : 0.f;
+		pr = kept ? weight * act_rgb(v[0], A.K.rgb_act) : 0.f; pg = kept ? weight * act_rgb(v[1], A.K.rgb_act) : 0.f; pb = kept ? weight * act_rgb(v[2], A.K.rgb_act) : 0.f;
 		s_was = s; T_was = T; alpha_was = alpha;
-		T_in = lane_f32(T * f, WAVE - 1u);
+		c.T = lane_f32(T * f, WAVE - 1u);
+		if (COUNT) n = end;
 	}
-	c.T = T_in; c.Cr = r_in; c.Cg = g_in; c.Cb = b_in;
 }
 
 constexpr uint32_t LONG_THREADS = 256;         // four independent wavefronts
 constexpr uint32_t LONG_WORKGROUPS = 2048;
 
+__device__ __forceinline__ fused::RayCarry walk_begin() { fused::RayCarry c; c.T = 1.f; c.Cr = 0.f; c.Cg = 0.f; c.Cb = 0.f; c.k = 0; c.numsteps = 0; c.done = 0; return c; }
+// samples of a stretch: whole blocks of 64, so many that LONG_STRETCHES cover the ray
+__device__ __forceinline__ uint32_t long_stretch(uint32_t numsteps) { return div_up(div_up(numsteps, WAVE), LONG_STRETCHES) * WAVE; }
+
+// the loop of one ray to its end, and the ray's colour (ray_marcher.cu:57-92); saved: its record for the backward walk, or NULL
+template <bool HALF_IN>
+__device__ __forceinline__ LongRay long_forward(uint32_t lane, const fused::Args& A, uint32_t i, uint32_t numsteps, uint32_t base, LongRay* saved) {
+	fused::RayCarry c = walk_begin();
+	const uint32_t stretch = long_stretch(numsteps);
+	LongRay R;
+	R.base = base;
+	R.n_fwd = walk<HALF_IN, true>(lane, A, base, 0u, numsteps, c, [](uint32_t, const WalkSample<HALF_IN>&, float, Float4) {}, [&](uint32_t k, const fused::RayCarry& now) {
+		if (saved && k % stretch == 0u && lane == 0) saved->at[k / stretch] = mk4(now.T, now.Cr, now.Cg, now.Cb);
+	});
+	float target[3], bg[3], loss;
+	target_and_background(A.K, *(const Float4*)(A.rays_rgba + 4 * (size_t)i), target, bg);
+	if (R.n_fwd == numsteps) { c.Cr += c.T * bg[0]; c.Cg += c.T * bg[1]; c.Cb += c.T * bg[2]; }
+	R.c[0] = c.Cr; R.c[1] = c.Cg; R.c[2] = c.Cb;
+	for (int k = 0; k < 3; ++k) loss_channel(A.K.loss_type, target[k], R.c[k], &loss, &R.g[k]);
+	if (saved && lane == 0) {
+		*(Float4*)&saved->g[0] = mk4(R.g[0], R.g[1], R.g[2], srf_u2f(R.n_fwd));
+		*(Float4*)&saved->c[0] = mk4(R.c[0], R.c[1], R.c[2], srf_u2f(R.base));
+		saved->stretch = stretch;
+	}
+	return R;
+}
+
 template <bool HALF_IN, bool HALF_OUT, bool BACKWARD>
 __global__ void __launch_bounds__(LONG_THREADS) k_long_rays(fused::Args A, const uint32_t* __restrict__ n_rays_counter, const float* __restrict__ mean_density_ptr, ChainScratch S) {
 	using namespace fused;
 	const uint32_t lane = threadIdx.x % WAVE;
-	// a unit of work: one ray of a listed group
-	const uint64_t n_units = (uint64_t)*S.slow_count * RAYS;
+	// a unit of work: one ray of a listed group, backward one stretch of it
+	constexpr uint32_t PARTS = BACKWARD ? LONG_STRETCHES : 1u;
+	const uint64_t n_units = (uint64_t)*S.slow_count * RAYS * PARTS;
 	uint64_t unit = (uint64_t)blockIdx.x * (LONG_THREADS / WAVE) + threadIdx.x / WAVE;
 	if (unit >= n_units) return;
 	const uint32_t counter_now = *n_rays_counter;
 	A.mean_density = mean_density_ptr ? *mean_density_ptr : 0.f;
 	A.n_active = counter_now < A.K.n_rays ? counter_now : A.K.n_rays;
 	for (; unit < n_units; unit += (uint64_t)gridDim.x * (LONG_THREADS / WAVE)) {
-		const uint32_t i = SRF_UNIFORM_U32(S.items[S.slow_items[unit / RAYS]].x * RAYS + (uint32_t)(unit % RAYS));
+		const uint32_t slot = SRF_UNIFORM_U32((uint32_t)(unit / PARTS)), part = SRF_UNIFORM_U32((uint32_t)(unit % PARTS));
+		const uint32_t i = SRF_UNIFORM_U32(S.items[S.slow_items[slot / RAYS]].x * RAYS + slot % RAYS);
 		if (i >= A.n_active) continue;
-		const U2 rec = *(const U2*)(A.ray_coord_indices + 2 * (size_t)i);
-		const uint32_t numsteps = SRF_UNIFORM_U32(rec.x), base = SRF_UNIFORM_U32(rec.y);
-		const uint32_t n_fwd = walk_count<HALF_IN>(lane, A, base, numsteps);
+		LongRay* saved = slot < LONG_SAVED ? (LongRay*)S.long_rays + slot : nullptr;
 		if (!BACKWARD) {
-			if (lane == 0) S.side[i] = n_fwd;
+			const U2 rec = *(const U2*)(A.ray_coord_indices + 2 * (size_t)i);
+			const LongRay R = long_forward<HALF_IN>(lane, A, i, SRF_UNIFORM_U32(rec.x), SRF_UNIFORM_U32(rec.y), saved);
+			if (lane == 0) {
+				S.side[i] = R.n_fwd;
+				if (A.rgb_ray_out) { A.rgb_ray_out[3 * (size_t)i] = R.c[0]; A.rgb_ray_out[3 * (size_t)i + 1] = R.c[1]; A.rgb_ray_out[3 * (size_t)i + 2] = R.c[2]; }
+			}
 			continue;
 		}
-		RayCarry c;
-		walk_colours<HALF_IN>(lane, A, base, n_fwd, c, [](uint32_t, const WalkSample<HALF_IN>&, float, Float4) {});
-		// finish_ray and commit_ray for one ray (ray_marcher.cu:81-133)
-		float target[3], bg[3];
-		target_and_background(A.K, *(const Float4*)(A.rays_rgba + 4 * (size_t)i), target, bg);
-		if (n_fwd == numsteps) { c.Cr += c.T * bg[0]; c.Cg += c.T * bg[1]; c.Cb += c.T * bg[2]; }
-		float lo[3];
-		Float4 og = mk4(0.f, 0.f, 0.f, 0.f);
-		loss_channel(A.K.loss_type, target[0], c.Cr, &lo[0], &og.x);
-		loss_channel(A.K.loss_type, target[1], c.Cg, &lo[1], &og.y);
-		loss_channel(A.K.loss_type, target[2], c.Cb, &lo[2], &og.z);
-		const uint32_t cbase = S.side[i];
+		if (!saved && part != 0u) continue;
+		const uint32_t cbase = SRF_UNIFORM_U32(S.side[i]);
+		Float4 og, oc;
+		uint32_t k_lo = 0u, k_hi = 0xffffffffu;
+		RayCarry c = walk_begin();
+		if (saved) {
+			// (not the ray's record, which the wavefront of its first stretch overwrites)
+			og = *(const Float4*)&saved->g[0]; oc = *(const Float4*)&saved->c[0];
+		} else {
+			const U2 rec = *(const U2*)(A.ray_coord_indices + 2 * (size_t)i);
+			const LongRay R = long_forward<HALF_IN>(lane, A, i, SRF_UNIFORM_U32(rec.x), SRF_UNIFORM_U32(rec.y), nullptr);
+			og = mk4(R.g[0], R.g[1], R.g[2], srf_u2f(R.n_fwd)); oc = mk4(R.c[0], R.c[1], R.c[2], srf_u2f(R.base));
+		}
+		const uint32_t n_fwd = SRF_UNIFORM_U32(srf_f2u(og.w)), base = SRF_UNIFORM_U32(srf_f2u(oc.w));
 		const uint32_t room = A.K.n_max_compacted - (A.K.n_max_compacted < cbase ? A.K.n_max_compacted : cbase);
 		const uint32_t n = room < n_fwd ? room : n_fwd;
-		if (lane == 0) {
-			if (A.rgb_ray_out) { A.rgb_ray_out[3 * (size_t)i] = c.Cr; A.rgb_ray_out[3 * (size_t)i + 1] = c.Cg; A.rgb_ray_out[3 * (size_t)i + 2] = c.Cb; }
+		if (part == 0u && lane == 0) {
+			// commit_ray and commit_loss for one ray (ray_marcher.cu:116-133)
 			A.ray_coord_indices[2 * (size_t)i] = n;
 			A.ray_coord_indices[2 * (size_t)i + 1] = cbase;
-			if (n != 0 && A.loss_output) A.loss_output[i] = (((lo[0] + lo[1]) + lo[2]) / 3.0f) / (float)A.K.n_rays;
+			if (n != 0 && A.loss_output) {
+				float target[3], bg[3], lo[3], g;
+				target_and_background(A.K, *(const Float4*)(A.rays_rgba + 4 * (size_t)i), target, bg);
+				loss_channel(A.K.loss_type, target[0], oc.x, &lo[0], &g);
+				loss_channel(A.K.loss_type, target[1], oc.y, &lo[1], &g);
+				loss_channel(A.K.loss_type, target[2], oc.z, &lo[2], &g);
+				A.loss_output[i] = (((lo[0] + lo[1]) + lo[2]) / 3.0f) / (float)A.K.n_rays;
+			}
 		}
-		const Float4 oc = mk4(c.Cr, c.Cg, c.Cb, 0.f);
-		walk_colours<HALF_IN>(lane, A, base, n, c, [&](uint32_t k, const WalkSample<HALF_IN>& s, float alpha, Float4 after) {
+		if (saved) {
+			// the stretches the forward walk was cut into went by the ray's length; it has left the loop's state for those it reached
+			const uint32_t stretch = SRF_UNIFORM_U32(saved->stretch);
+			k_lo = part * stretch; k_hi = k_lo + stretch;
+			if (k_lo >= n) continue;
+			const Float4 at = saved->at[part];
+			c.T = at.x; c.Cr = at.y; c.Cg = at.z; c.Cb = at.w;
+		}
+		const uint32_t end = k_hi < n ? k_hi : n;
+		walk<HALF_IN, false>(lane, A, base, k_lo, end, c, [&](uint32_t k, const WalkSample<HALF_IN>& s, float alpha, Float4 after) {
 			float v[4];
 			unpack_raw<HALF_IN>(s.raw, v);
 			sample_gradient<HALF_OUT, false>(A, v, s.dt, alpha, after, og, oc, (size_t)cbase + k);
-		});
+		}, [](uint32_t, const RayCarry&) {});
 		if (A.compacted_coords) {
 			const float* src = A.coords + 7 * (size_t)base;
 			float* dst = A.compacted_coords + 7 * (size_t)cbase;
-			for (uint32_t k = lane; k < 7u * n; k += WAVE) dst[k] = src[k];
+			for (size_t k = 7 * (size_t)k_lo + lane; k < 7 * (size_t)end; k += WAVE) dst[k] = src[k];
 		}
 	}
 }

@@ -1,0 +1,62 @@
+"""Training compositing of rays that have a wavefront to themselves, against the oracle: lengths round a block of 64 samples, round
+the length from which a group of rays goes that way and far beyond it, rays that end early in any block, a capacity that clamps
+inside a long ray, more such rays than the forward walk keeps a record for (their backward walk begins anew), with and without records."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from tests import helpers
+from tests.test_gpu_parity import u32
+from tests.test_oracle_composite import loss_args
+
+pytestmark = pytest.mark.gpu
+LENGTHS = [0, 1, 63, 64, 65, 127, 128, 129, 191, 255, 256, 257, 511, 512, 513, 1024, 1920, 2042, 5000]
+
+
+@pytest.mark.parametrize("hin,hout", [(True, True), (False, False)])
+@pytest.mark.parametrize("kind", ["lengths", "one_a_group", "early_end", "many_listed", "clamped"])
+def test_long_rays_against_the_oracle(gpu, orc, kind, hin, hout):
+    torch = gpu
+    from sphericalrf_amd import api
+    rng = np.random.default_rng(len(kind))
+    n_rays = 64 * 600 + 5 if kind == "many_listed" else 64 * 6 + 13
+    if kind == "many_listed":
+        counts = rng.integers(0, 30, n_rays)
+    elif kind == "one_a_group":
+        counts = rng.integers(0, 40, n_rays)
+        counts[::64] = [LENGTHS[-1 - k] for k in range(len(counts[::64]))]
+    else:
+        counts = rng.choice(LENGTHS, n_rays)
+    base = np.concatenate([[0], np.cumsum(counts)[:-1]])
+    total = int(counts.sum())
+    if kind == "many_listed":                     # offsets in no order: every group is listed
+        order = rng.permutation(n_rays)
+        base[order] = np.concatenate([[0], np.cumsum(counts[order])[:-1]])
+    net = helpers.random_network_output(rng, total, np.float16 if hin else np.float32)
+    net[:, 3] *= net.dtype.type(2.0 if kind == "early_end" else 0.02)
+    coords = rng.random((total, 7)).astype(np.float32)
+    coords[:, 3] = coords[:, 3] * 0.3 + 0.01
+    tgt = rng.random((n_rays, 4)).astype(np.float32)
+    cap = int(total * (0.4 if kind == "clamped" else 1.0)) + 1
+    act = dict(rgb_activation=O.ACT_LOGISTIC, density_activation=O.ACT_NONE) if hin else {}
+    a = loss_args(n_rays, cap, network_output_dtype=O.DTYPE_F16 if hin else O.DTYPE_F32, dloss_dtype=O.DTYPE_F16 if hout else O.DTYPE_F32, dt_stride=7,
+                  background_color=(O.f32 * 3)(0.3, 0.5, 0.7), mean_density=0.001, **act)
+    idx = np.stack([counts, base], axis=1).astype(np.uint32)
+    o_idx, o_dloss = idx.copy(), np.zeros((cap, 4), np.float16 if hout else np.float32)
+    o_comp, o_loss, o_rgb = np.zeros((cap, 7), np.float32), np.full(n_rays, -1, np.float32), np.zeros((n_rays, 3), np.float32)
+    o_total = orc.volume_rendering_with_loss_and_gradient(a, tgt, n_rays - 3, o_idx, coords.ravel()[3:], net, o_dloss, n_compacted_counter=2, coords=coords,
+                                                          compacted_coords=o_comp, loss_output=o_loss, rgb_ray_out=o_rgb)
+    m = api.RayMarcher(dict(train_with_random_bg_color=False, train_in_linear_color=True, transmittance_threshold=1e-4))
+    d_coords, d_idx = torch.from_numpy(coords).cuda(), torch.from_numpy(idx.view(np.int32)).cuda()
+    d_dloss = torch.zeros((cap, 4), dtype=torch.float16 if hout else torch.float32, device="cuda")
+    d_comp, d_loss, d_rgb = torch.zeros((cap, 7), device="cuda"), torch.full((n_rays,), -1.0, device="cuda"), torch.zeros((n_rays, 3), device="cuda")
+    cnt, nrc = torch.full((1,), 2, dtype=torch.int32, device="cuda"), torch.full((1,), n_rays - 3, dtype=torch.int32, device="cuda")
+    m.volume_rendering_with_loss_and_gradient(n_rays, cap, torch.from_numpy(tgt).cuda(), nrc, d_idx, d_coords.view(-1)[3:], torch.from_numpy(net).cuda(), d_dloss, cnt,
+                                              rgb_activation=api.ACT_LOGISTIC if hin else api.ACT_NONE, density_activation=api.ACT_NONE, loss_output=d_loss, loss_type="L2",
+                                              loss_scale=128.0, density_grid_mean=torch.full((1,), 0.001, device="cuda"), background_color=(0.3, 0.5, 0.7), coords=d_coords,
+                                              compacted_coords=d_comp, dt_stride=7, rgb_ray_out=d_rgb)
+    m.sync_check()
+    assert int(cnt.item()) == o_total and np.array_equal(u32(d_idx), o_idx)
+    assert np.array_equal(d_rgb.cpu().numpy().view(np.uint32), o_rgb.view(np.uint32)) and np.array_equal(d_loss.cpu().numpy().view(np.uint32), o_loss.view(np.uint32))
+    bits = np.uint16 if hout else np.uint32
+    assert np.array_equal(d_dloss.cpu().numpy().view(bits), o_dloss.view(bits)) and np.array_equal(d_comp.cpu().numpy(), o_comp)
