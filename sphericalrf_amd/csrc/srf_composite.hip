@@ -50,11 +50,12 @@ __global__ void __launch_bounds__(128) k_volume_rendering(Params P, srf_render_a
 constexpr uint32_t LONG_RAY = 128;
 // What the forward walk of a long ray leaves: the gradient of the loss, how many samples the ray consumes, its colour, its first
 // sample, and where the loop stands at the beginning of each of eight stretches {transmittance, colour sum}, which the backward walk
-// then takes side by side.  Kept for the first LONG_SAVED rays; with more, the others' stretches would have to wait anyway, and the
-// backward walk of such a ray begins from its first sample.
+// then takes side by side.  Kept for the first LONG_SAVED rays, the initial batch of a training; with more, the others' stretches would
+// have to wait anyway, and the backward walk of such a ray begins from its first sample.  (A record is 176 bytes, and a caller's
+// first call allocates them: 32768 made that call 0.25 to 0.5 ms longer.)
 constexpr uint32_t LONG_STRETCHES = 8;
 struct alignas(16) LongRay { float g[3]; uint32_t n_fwd; float c[3]; uint32_t base; uint32_t stretch, pad[3]; Float4 at[LONG_STRETCHES]; };
-constexpr uint32_t LONG_SAVED = 32768;
+constexpr uint32_t LONG_SAVED = 4096;
 
 // bytes of device scratch the chain needs for n_rays rays whose groups are cut into at most max_parts items each, and where
 // its parts lie
