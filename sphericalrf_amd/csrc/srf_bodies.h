@@ -1138,6 +1138,22 @@ SRF_HD void field_eval_body(uint32_t i, const Params& P, const float* coords, co
 	net_store<HALF>(out, (size_t)i * width + 3, row.w);
 }
 
+// colour and opacity of an occupied sample
+SRF_HD Float4 fused_sample(const Params& P, const FieldArgs& F, const Probe& s) {
+	Float4 row = *(const Float4*)(F.table + 4 * (size_t)field_row(P, s.w, F));
+	row.w = 1.f - srf_expf(-row.w * s.dt);
+	return row;
+}
+// true when the ray is opaque with it
+SRF_HD bool fused_composite(Float4 sample, float thr, Float4& acc, uint32_t& count) {
+	const float T = 1.f - acc.w;
+	const float weight = sample.w * T;
+	acc.x += sample.x * weight; acc.y += sample.y * weight; acc.z += sample.z * weight;
+	acc.w += weight;
+	++count;
+	return acc.w > (1.0f - thr);
+}
+
 // Whole-frame render: the ray of a pixel is generated, advanced and marched to the
 // end, compositing every occupied sample as volume_rendering_kernel does
 // (ray_marcher.cu:233-273) and finishing with shade_kernel's store (testbed.cu:448-477)
@@ -1154,14 +1170,7 @@ struct FusedMarch {
 		const Params* P; const FieldArgs* F; float thr; Float4* acc; uint32_t* count;
 		SRF_HD MarchEnd operator()(MarchLane& L, const Probe& s) const {
 			if (s.dt == 0.f) { *acc = mk4(0.f, 0.f, 0.f, 0.f); return MARCH_STOPPED; }
-			const Float4 row = *(const Float4*)(F->table + 4 * (size_t)field_row(*P, s.w, *F));
-			const float T = 1.f - acc->w;
-			const float alpha = 1.f - srf_expf(-row.w * s.dt);
-			const float weight = alpha * T;
-			acc->x += row.x * weight; acc->y += row.y * weight; acc->z += row.z * weight;
-			acc->w += weight;
-			++*count;
-			if (acc->w > (1.0f - thr)) return MARCH_STOPPED;
+			if (fused_composite(fused_sample(*P, *F, s), thr, *acc, *count)) return MARCH_STOPPED;
 			L.t += s.dt;
 			L.phase = LANE_PROBE;
 			return MARCH_GOES_ON;

@@ -722,7 +722,9 @@ int srf_sampler_create(const srf_sampler_config* c, srf_sampler_t** out) {
 	{ const char* v = getenv("SRF_SPLAT_SORT"); if (v && v[0] == '2') s->force_splat_sort = 2; }      // 2: large-batch path through the library's sort
 	s->force_sample_bits = tri_state("SRF_GRID_SAMPLE_BITS");
 	s->force_sample_by_cell = tri_state("SRF_GRID_SAMPLE_BY_CELL");
-	{ const char* v = getenv("SRF_COUNT_TEAM"); const uint32_t n = v && v[0] ? (uint32_t)atoi(v) : 0u; s->count_team = is_pow2(n) && n <= 64u ? n : 0u; }
+	auto team_size = [](const char* name) { const char* v = getenv(name); const uint32_t n = v && v[0] ? (uint32_t)atoi(v) : 0u; return is_pow2(n) && n <= 64u ? n : 0u; };
+	s->count_team = team_size("SRF_COUNT_TEAM");
+	s->march_team = team_size("SRF_MARCH_TEAM");
 	// SRF_MARCH_PARK_ALL=1: the render marches hand every ray that finds an empty cell without anything to skip to their
 	// one-ray-per-wavefront march at once, whatever the wavefront still holds (for tests: that march then does most of a frame)
 	{ const char* v = getenv("SRF_MARCH_PARK_ALL"); s->march_park_all = v && v[0] == '1'; }

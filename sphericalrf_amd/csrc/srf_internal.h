@@ -56,7 +56,7 @@ struct srf_sampler {
 	// Switches the tests use to run both sides of a size-dependent choice on small inputs; read from the environment once, when the
 	// sampler is created (-1: the library chooses): SRF_SPLAT_SORT, SRF_GRID_SAMPLE_BITS, SRF_GRID_SAMPLE_BY_CELL = 0|1
 	// (SRF_SPLAT_SORT=2: the large-batch splat through the library's radix sort instead of the partition made for it);
-	// SRF_COUNT_TEAM = lanes a ray of the counting march begins with (a power of two up to 64)
+	// SRF_COUNT_TEAM, SRF_MARCH_TEAM = lanes a ray of the counting march, of the render marches begins with (a power of two up to 64)
 	int      force_splat_sort, force_sample_bits, force_sample_by_cell;
 	uint32_t count_team = 0;
 	bool     grid_sample_cell_order = false;   // srf_sampler_set_grid_sample_order
@@ -66,6 +66,7 @@ struct srf_sampler {
 	uint32_t* park_counts = nullptr; // two counters of that queue, used in turn: a march clears the one the next march will use
 	uint32_t park_turn = 0;
 	bool march_park_all = false;     // SRF_MARCH_PARK_ALL at creation
+	uint32_t march_team = 0;         // SRF_MARCH_TEAM
 };
 
 struct srf_marcher {

@@ -366,8 +366,8 @@ __global__ void __launch_bounds__(128) k_init_rays(Params P, PixelArgs A, srf_ra
 	if (x < (uint32_t)A.res[0] && y < (uint32_t)A.res[1]) init_ray_body(x, y, P, A, payloads);
 }
 
-// The render marches (first occupied cell, next chunk of samples, whole frame), one wavefront per block and one ray per
-// lane.  Every round the wavefront runs one phase of srf_bodies.h's march machine: steps through known-empty space while
+// The render marches (first occupied cell, next chunk of samples, whole frame) of many rays, one wavefront per block and one ray per
+// lane (of few rays: k_march_teams below).  Every round the wavefront runs one phase of srf_bodies.h's march machine: steps through known-empty space while
 // any lane has some to take, a grid probe (with whatever the march does at an occupied cell) once all lanes wait for one.
 // A lane waiting for its probe idles through the step rounds, so that the expensive probe is issued for all lanes at once.
 // Letting the probing lanes go first once they outnumber the stepping ones, and stepping in bursts of a fixed length (as the
@@ -519,10 +519,195 @@ __global__ void __launch_bounds__(64) k_march_lanes(March M, MarchPark park) {
 #endif
 }
 
-// the march and, behind it, the wide march of the rays it parked
+// What a team's probe knows of its steps: bit k of the masks is the team's k-th step, starts[k] the t it begins with, t_end the t
+// behind the last one; `own` is the probe of this lane's step.
+struct TeamSteps { uint32_t sub, team; const float* starts; float t_end; uint64_t occ; bool zero; Probe own; };
+__device__ __forceinline__ float team_step_end(const TeamSteps& S, uint32_t k) { return k + 1u < S.team ? S.starts[k + 1u] : S.t_end; }
+
+// What the occupied ones of a team's steps do to its ray, in step order; every lane of the team holds the ray's state.
+__device__ __forceinline__ MarchEnd team_hits(const AdvanceMarch&, AdvanceMarch::Lane& L, const TeamSteps& S, Float4*, uint64_t) {
+	if (!S.occ) return MARCH_GOES_ON;
+	L.m.t = S.starts[__builtin_ctzll(S.occ)];
+	return MARCH_STOPPED;
+}
+__device__ __forceinline__ MarchEnd team_hits(const CoordsMarch& M, CoordsMarch::Lane& L, const TeamSteps& S, Float4*, uint64_t) {
+	const uint32_t rank = (uint32_t)__popcll(S.occ & low_bits64(S.sub)), found = (uint32_t)__popcll(S.occ), room = M.n_steps - L.j;
+	if (((S.occ >> S.sub) & 1ull) != 0ull && rank < room) {
+		float* q = M.coords + 7 * ((size_t)L.i * M.n_steps + (L.j + rank));
+		st3(q, S.own.w); q[3] = S.own.dt; st3(q + 4, L.wdir);
+	}
+	if (found < room) { L.j += found; return MARCH_GOES_ON; }
+	uint64_t m = S.occ;
+	for (uint32_t k = 1; k < room; ++k) m &= m - 1ull;
+	L.m.t = team_step_end(S, (uint32_t)__builtin_ctzll(m));
+	L.j = M.n_steps;
+	return MARCH_STOPPED;
+}
+// (rows: one of LDS a lane of the team; zero: which of the steps are of size zero)
+__device__ __forceinline__ MarchEnd team_hits(const FusedMarch& M, FusedMarch::Lane& L, const TeamSteps& S, Float4* rows, uint64_t zero) {
+	for (uint64_t m = S.occ; m; m &= m - 1ull) {
+		const uint32_t k = (uint32_t)__builtin_ctzll(m);
+		if ((zero >> k) & 1ull) { L.acc = mk4(0.f, 0.f, 0.f, 0.f); return MARCH_STOPPED; }
+		if (fused_composite(rows[k], M.thr, L.acc, L.count)) return MARCH_STOPPED;
+	}
+	return MARCH_GOES_ON;
+}
+// what a lane prepares for team_hits where its step is occupied: colour and opacity of its sample
+template <class March> __device__ __forceinline__ void team_row(const March&, const TeamSteps&, Float4*) {}
+__device__ __forceinline__ void team_row(const FusedMarch& M, const TeamSteps& S, Float4* row) { *row = fused_sample(M.G.P, M.F, S.own); }
+
+// count_team_probe for the render marches
+template <class March>
+__device__ __forceinline__ MarchEnd march_team_probe(const March& M, typename March::Lane& lane_state, uint32_t team, float* starts, Float4* rows) {
+	const Params& P = M.G.P;
+	MarchLane& L = lane_state.m;
+	const uint32_t lane = threadIdx.x & 63u, sub = lane & (team - 1u), lead = lane - sub;
+	const float cone = P.cone_angle_constant;
+	const bool mine = L.phase == LANE_PROBE;
+	const ShortForm f = disparity_short_form(P);
+	const bool chains = f.usable && mine && L.t >= f.t_lo;
+	ShortChain ch = short_chain_at(chains ? L.t : 1.f);
+	TeamSteps S;
+	S.sub = sub; S.team = team; S.starts = starts + lead; S.zero = false;
+	float t_mine = L.t;
+	for (uint32_t k = 0; k < team; ++k) {
+		t_mine = k == sub ? ch.t : t_mine;
+		ch = short_chain_next(f, ch);
+	}
+	S.t_end = ch.t;
+	// every step has to start inside the short form's range; a team with one that does not goes through calc_dt
+	const uint64_t outside_form = __ballot(!chains || !(t_mine >= f.t_lo && t_mine <= f.t_hi));
+	if (mine && (outside_form & (low_bits64(team) << lead)) != 0ull) {
+		float t = L.t;
+		for (uint32_t k = 0; k < team; ++k) {
+			const float dt = calc_dt(P, t, cone);
+			if (k == sub) { t_mine = t; S.zero = dt == 0.f; }
+			t += dt;
+		}
+		S.t_end = t;
+	}
+	bool inside = false, occupied = false;
+	float limit = t_mine;
+	if (mine) {
+		const Vec3 pos = along(L.o, L.d, t_mine);
+		inside = aabb_contains(P, pos);
+		bool look = inside;
+		if (inside && P.sphere[3] > 0.f) {
+			float t_enter;
+			const SphereGate g = sphere_gate(P, L.o, L.d, t_mine, &t_enter);
+			if (g == SPHERE_BEYOND) inside = look = false;
+			if (g == SPHERE_BEFORE) { look = false; limit = t_enter; }
+		}
+		if (look) {
+			S.own = probe_at(P, M.G.bitfield, pos, t_mine, cone, &M.G.skip);
+			occupied = S.own.occ;
+			if (occupied) team_row(M, S, rows + lane);
+			else if (M.G.skipping()) limit = skip_limit(P, M.G.skip, L.sr, L.o, L.d, t_mine, S.own.radius, S.own.level);
+		}
+	}
+	const uint64_t all = low_bits64(team);
+	const uint64_t m_inside = __ballot(inside) >> lead, m_occ = __ballot(occupied) >> lead, m_zero = __ballot(S.zero) >> lead;
+	starts[lane] = t_mine;
+	limit = __shfl(limit, (int)(lead + team - 1u), 64);
+	__syncthreads();
+	MarchEnd end = MARCH_GOES_ON;
+	if (mine) {
+		// the march ends at the first step that is outside or, its cell being empty, of size zero
+		const uint64_t m_end = (~m_inside | (m_zero & ~m_occ)) & all;
+		const uint32_t n = m_end ? (uint32_t)__builtin_ctzll(m_end) : team;
+		S.occ = m_occ & low_bits64(n);
+		end = team_hits(M, lane_state, S, rows + lead, m_zero);
+		if (end == MARCH_GOES_ON) {
+			if (m_end) {
+				L.t = S.starts[n];
+				end = ((m_inside >> n) & 1ull) == 0ull ? MARCH_LEFT_BOX : MARCH_ZERO_STEP;
+			} else {
+				L.t = S.t_end;
+				L.t_limit = limit;
+				L.phase = L.t < L.t_limit ? LANE_STEP : LANE_PROBE;
+			}
+		}
+	}
+	__syncthreads();
+	return end;
+}
+
+// the state of the ray in lane `from`
+template <class Lane>
+__device__ __forceinline__ void march_move(Lane& L, uint32_t from) {
+	uint32_t w[sizeof(Lane) / 4];
+	__builtin_memcpy(w, &L, sizeof(Lane));
+	#pragma unroll
+	for (uint32_t k = 0; k < sizeof(Lane) / 4; ++k) w[k] = moved(w[k], from);
+	__builtin_memcpy(&L, w, sizeof(Lane));
+}
+
+// A launch of few rays, by teams of lanes.  Bound by one ray's probes waiting for one another: a preview of 64 x 64 pixels is 64
+// wavefronts with a ray a lane, each as long as its longest ray.  As in the counting march, a ray is therefore worked on by a team of lanes that
+// looks its next steps up side by side, and a wavefront whose rays left fill half of its lanes at most gathers them and gives each
+// more lanes.  What a march does at occupied cells is then done for the team's steps in their order (team_hits).
+// Measured against a ray a lane with the crawling rays on wavefronts of their own behind it (us a frame, three cameras each): 64 x 64 pixels of
+// the 64^3 grid 790 / 425 / 95 -> 100 / 93 / 53, 256 x 256 857 / 447 / 95 -> 358 / 245 / 90, 160 x 120 of the five-cascade
+// grid 312 / 206 / 195 -> 143 / 128 / 122.
+// Lanes a ray begins with: as many as keep the launch at 2^18 lanes, 32 at most (160 x 120 pixels, lanes a ray -> us, 64^3 / five
+// cascades: 2: 552 / 225, 4: 314 / 169, 8: 181 / 143, 16: 162 / 164, 32: 207 / 251; 64 x 64: 8: 163 / 126, 16: 119 / 108, 32: 100 / 103, 64: 103 / 127).
+// With more rays than leave each two lanes the chip is full of rays and the march above is the faster one: a team's round takes more
+// registers (five wavefronts a SIMD instead of six) and looks cells up ahead of their time (1920 x 1080 pixels of the five
+// cascades 1070 -> 1153 us, 1024 x 768 of the bounded object 711 -> 982 us).
+constexpr uint64_t MARCH_LANES = 262144;
+constexpr uint32_t MARCH_TEAM_MAX = 32;
+template <class March>
+__global__ void __launch_bounds__(64) k_march_teams(March M, uint32_t team) {
+	__shared__ float starts[64];
+	__shared__ uint32_t from_lane[64];
+	__shared__ Float4 rows[64];
+	march_resolve(M);
+	const uint32_t lane = threadIdx.x;
+	const uint32_t q = blockIdx.x * (64u / team) + lane / team;
+	typename March::Lane L;
+	L.m.phase = LANE_IDLE;
+	MarchEnd end = q < M.lanes() ? M.begin(L, q) : MARCH_NO_RAY;
+	for (;;) {
+		if (end != MARCH_GOES_ON) {
+			if (end != MARCH_NO_RAY && (lane & (team - 1u)) == 0u) M.finish(L, end);
+			L.m.phase = LANE_IDLE;
+			end = MARCH_GOES_ON;
+		}
+		const uint64_t m_probe = __ballot(L.m.phase == LANE_PROBE), m_step = __ballot(L.m.phase == LANE_STEP);
+		uint32_t alive = (uint32_t)__popcll(m_probe | m_step);
+		if (!alive) break;
+		if (m_step) {
+			if (L.m.phase == LANE_STEP) end = M.steps(L);
+		} else if (alive <= 32u && team < 64u) {
+			uint32_t larger = team;
+			while (alive * 2u <= 64u && larger < 64u) { larger *= 2u; alive *= 2u; }
+			const uint64_t m_lead = __ballot(L.m.phase == LANE_PROBE && (lane & (team - 1u)) == 0u);
+			if ((m_lead >> lane) & 1ull) from_lane[__popcll(m_lead & low_bits64(lane))] = lane;
+			__syncthreads();
+			const uint32_t ray = lane / larger;
+			const bool takes = ray < (uint32_t)__popcll(m_lead);
+			march_move(L, takes ? from_lane[ray] : 0u);
+			if (!takes) L.m.phase = LANE_IDLE;
+			team = larger;
+			__syncthreads();
+		} else {
+			end = march_team_probe(M, L, team, starts, rows);
+		}
+	}
+}
+
+// the march; with a ray a lane, behind it the wide march of the rays it parked
 template <class March>
 static int launch_march(const March& M, srf_sampler* s, hipStream_t st) {
 	const uint32_t n = M.lanes();
+	uint32_t team = 1;
+	while (team < MARCH_TEAM_MAX && (uint64_t)n * team * 2u <= MARCH_LANES) team *= 2u;
+	if (s->march_team) team = s->march_team;
+	if (team > 1u && !s->march_park_all) {
+		hipLaunchKernelGGL(k_march_teams<March>, dim3(div_up(n, 64u / team)), dim3(64), 0, st, M, team);
+		SRF_LAUNCH_CHECK();
+		return SRF_OK;
+	}
 	MarchPark park;
 	park.capacity = s->march_park_all ? n : n / 8u + 64u;
 	park.max_lanes = s->march_park_all ? 64u : PARK_MAX_LANES;
