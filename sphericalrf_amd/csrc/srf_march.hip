@@ -656,6 +656,15 @@ __device__ __forceinline__ void march_move(Lane& L, uint32_t from) {
 // cascades 1070 -> 1153 us, 1024 x 768 of the bounded object 711 -> 982 us).
 constexpr uint64_t MARCH_LANES = 262144;
 constexpr uint32_t MARCH_TEAM_MAX = 32;
+// The march to a loop's next samples goes this way with a ray a lane too: its rays are few and scattered once most pixels are
+// finished, whatever the frame's size, and gathering the last ones of a wavefront pays there (1920 x 1080 pixels of the five
+// cascades by the loop 5.82 -> 5.14 ms, 1024 x 768 3.77 -> 3.13 ms).
+template <class March> constexpr bool TEAMS_AT_ANY_SIZE = false;
+template <> constexpr bool TEAMS_AT_ANY_SIZE<CoordsMarch> = true;
+// Probes that a wavefront makes with half of its lanes at work before its rays are gathered: most rays end within a few, and
+// gathering costs a state's worth of lane shuffles (0 -> 4: 64 x 64 pixels of the 64^3 grid 55 -> 47 us, 160 x 120 of the five
+// cascades 126 -> 116 us; 8 and 16 the same there, and the loop's frames lose again what gathering gave them).
+constexpr uint32_t MARCH_PATIENCE = 4;
 template <class March>
 __global__ void __launch_bounds__(64) k_march_teams(March M, uint32_t team) {
 	__shared__ float starts[64];
@@ -667,6 +676,7 @@ __global__ void __launch_bounds__(64) k_march_teams(March M, uint32_t team) {
 	typename March::Lane L;
 	L.m.phase = LANE_IDLE;
 	MarchEnd end = q < M.lanes() ? M.begin(L, q) : MARCH_NO_RAY;
+	uint32_t sparse = 0;
 	for (;;) {
 		if (end != MARCH_GOES_ON) {
 			if (end != MARCH_NO_RAY && (lane & (team - 1u)) == 0u) M.finish(L, end);
@@ -678,7 +688,8 @@ __global__ void __launch_bounds__(64) k_march_teams(March M, uint32_t team) {
 		if (!alive) break;
 		if (m_step) {
 			if (L.m.phase == LANE_STEP) end = M.steps(L);
-		} else if (alive <= 32u && team < 64u) {
+		} else if (alive <= 32u && team < 64u && sparse++ >= MARCH_PATIENCE) {
+			sparse = 0;
 			uint32_t larger = team;
 			while (alive * 2u <= 64u && larger < 64u) { larger *= 2u; alive *= 2u; }
 			const uint64_t m_lead = __ballot(L.m.phase == LANE_PROBE && (lane & (team - 1u)) == 0u);
@@ -691,7 +702,8 @@ __global__ void __launch_bounds__(64) k_march_teams(March M, uint32_t team) {
 			team = larger;
 			__syncthreads();
 		} else {
-			end = march_team_probe(M, L, team, starts, rows);
+			if (team > 1u) end = march_team_probe(M, L, team, starts, rows);
+			else if (L.m.phase == LANE_PROBE) end = M.probe(L);
 		}
 	}
 }
@@ -703,7 +715,8 @@ static int launch_march(const March& M, srf_sampler* s, hipStream_t st) {
 	uint32_t team = 1;
 	while (team < MARCH_TEAM_MAX && (uint64_t)n * team * 2u <= MARCH_LANES) team *= 2u;
 	if (s->march_team) team = s->march_team;
-	if (team > 1u && !s->march_park_all) {
+	const bool teams = team > 1u || (TEAMS_AT_ANY_SIZE<March> && s->march_team != 1u);
+	if (teams && !s->march_park_all) {
 		hipLaunchKernelGGL(k_march_teams<March>, dim3(div_up(n, 64u / team)), dim3(64), 0, st, M, team);
 		SRF_LAUNCH_CHECK();
 		return SRF_OK;
