@@ -172,66 +172,60 @@ SRF_HD bool mask_camera_sees(const float* m, Vec3 p, float radius, float focal_x
 // The ten candidate cells do not depend on what the grid holds, so BATCH of them (1, 2, 5 or 10) are looked up side by side;
 // the first that passes, in the reference's order, is taken, the tenth if none does.  One dependent lookup after the other
 // makes a wavefront wait for its unluckiest lane, a memory round trip per try.
+SRF_HD uint32_t grid_sample_hash(uint32_t i, uint32_t n_elements, uint32_t step, uint32_t j) { return (i + step * n_elements) * 56924617u + 96925573u + j * 19349663u; }
+// the cell of a point's try j.  The remainder by the cell count is a mask when that is a power of two (every grid the library accepts
+// for ERP has one; an integer division costs some forty instructions, and there are up to ten here).
+template <bool POW2>
+SRF_HD uint32_t grid_sample_cell(uint32_t i, const Params& P, uint32_t n_elements, uint32_t step, uint32_t j) {
+	const uint32_t h = grid_sample_hash(i, n_elements, step, j);
+	return POW2 ? (h & (P.n_cells - 1u)) : (h % P.n_cells);
+}
+// which try is taken
 template <bool POW2, uint32_t BATCH>
-SRF_HD void grid_sample_tries_batched(uint32_t i, const Params& P, uint32_t n_elements, uint32_t step, uint32_t level, const float* grid_in, float thresh,
-                                      const uint32_t* above, uint32_t* cell_out, uint32_t* idx_out, const uint32_t* above_summary = nullptr) {
+SRF_HD uint32_t grid_sample_tries_batched(uint32_t i, const Params& P, uint32_t n_elements, uint32_t step, uint32_t level, const float* grid_in, float thresh,
+                                          const uint32_t* above, const uint32_t* above_summary = nullptr) {
 	static_assert(10 % BATCH == 0, "whole batches");
-	uint32_t cell = 0, idx = 0;
+	uint32_t taken = 9;
 	bool found = false;
-	const uint32_t h0 = (i + step * n_elements) * 56924617u + 96925573u;
 	for (uint32_t j0 = 0; j0 < 10 && !found; j0 += BATCH) {
-		uint32_t c[BATCH], id[BATCH];
 		bool pass[BATCH];
 #if defined(__HIP_DEVICE_COMPILE__)
 		#pragma unroll
 #endif
 		for (uint32_t q = 0; q < BATCH; ++q) {
-			const uint32_t h = h0 + (j0 + q) * 19349663u;
-			c[q] = POW2 ? (h & (P.n_cells - 1u)) : (h % P.n_cells);
-			id[q] = c[q] + level * P.n_cells;
+			const uint32_t id = grid_sample_cell<POW2>(i, P, n_elements, step, j0 + q) + level * P.n_cells;
 			// above_summary: one bit per word of `above`, set where the word has a cell that fails: a table small enough for the
 			// nearest cache, and where hardly any cell fails (the uniform draw: only masked cells do) it answers nearly every lookup
-			const uint32_t word = id[q] >> 5;
+			const uint32_t word = id >> 5;
 			if (above_summary && ((above_summary[word >> 5] >> (word & 31u)) & 1u) == 0u) pass[q] = true;
-			else pass[q] = above ? ((above[word] >> (id[q] & 31u)) & 1u) != 0u : grid_in[id[q]] > thresh;
+			else pass[q] = above ? ((above[word] >> (id & 31u)) & 1u) != 0u : grid_in[id] > thresh;
 		}
 #if defined(__HIP_DEVICE_COMPILE__)
 		#pragma unroll
 #endif
 		for (uint32_t q = 0; q < BATCH; ++q) {
-			if (!found) { cell = c[q]; idx = id[q]; found = pass[q]; }
+			if (!found && pass[q]) { taken = j0 + q; found = true; }
 		}
 	}
-	*cell_out = cell;
-	*idx_out = idx;
+	return taken;
 }
 template <bool POW2>
-SRF_HD void grid_sample_tries(uint32_t i, const Params& P, uint32_t n_elements, uint32_t step, uint32_t level, const float* grid_in, float thresh,
-                              const uint32_t* above, uint32_t tries_at_once, uint32_t* cell_out, uint32_t* idx_out, const uint32_t* above_summary = nullptr) {
-	if (tries_at_once >= 10u) grid_sample_tries_batched<POW2, 10>(i, P, n_elements, step, level, grid_in, thresh, above, cell_out, idx_out, above_summary);
-	else if (tries_at_once >= 5u) grid_sample_tries_batched<POW2, 5>(i, P, n_elements, step, level, grid_in, thresh, above, cell_out, idx_out, above_summary);
-	else if (tries_at_once >= 2u) grid_sample_tries_batched<POW2, 2>(i, P, n_elements, step, level, grid_in, thresh, above, cell_out, idx_out, above_summary);
-	else grid_sample_tries_batched<POW2, 1>(i, P, n_elements, step, level, grid_in, thresh, above, cell_out, idx_out, above_summary);
+SRF_HD uint32_t grid_sample_tries(uint32_t i, const Params& P, uint32_t n_elements, uint32_t step, uint32_t level, const float* grid_in, float thresh,
+                                  const uint32_t* above, uint32_t tries_at_once, const uint32_t* above_summary = nullptr) {
+	if (tries_at_once >= 10u) return grid_sample_tries_batched<POW2, 10>(i, P, n_elements, step, level, grid_in, thresh, above, above_summary);
+	if (tries_at_once >= 5u) return grid_sample_tries_batched<POW2, 5>(i, P, n_elements, step, level, grid_in, thresh, above, above_summary);
+	if (tries_at_once >= 2u) return grid_sample_tries_batched<POW2, 2>(i, P, n_elements, step, level, grid_in, thresh, above, above_summary);
+	return grid_sample_tries_batched<POW2, 1>(i, P, n_elements, step, level, grid_in, thresh, above, above_summary);
 }
 
-// above: optional table of the comparison grid_in[idx] > thresh, one bit per cell (bit idx & 31 of word idx >> 5),
-// 32 times smaller than the grid, so that the random lookups below mostly stay in the caches
-SRF_HD void grid_sample_point(uint32_t i, const Params& P, uint32_t n_elements, Pcg32 rng, uint32_t step,
-                              const float* grid_in, float thresh, Vec3* position, uint32_t* index, const uint32_t* above = nullptr,
-                              const PcgSkip* skip = nullptr, uint32_t tries_at_once = 1,
-                             const uint64_t* skip16_m = nullptr, const uint64_t* skip16_p = nullptr, const uint32_t* above_summary = nullptr) {
-	if (skip16_m) pcg_advance_skip16(rng, i * 4u, skip16_m, skip16_p);
-	else if (skip) pcg_advance_u32(rng, i * 4u, *skip);
-	else pcg_advance(rng, (uint64_t)(uint32_t)(i * 4u));
-	// (uint32_t)(f * C) % C with f in [0, 1): the product is at most C, so the remainder only matters when it is C itself
+// the first number drawn for a point says its cascade.  (uint32_t)(f * C) % C with f in [0, 1): the product is at most C, so the
+// remainder only matters when it is C itself
+SRF_HD uint32_t grid_sample_level(const Params& P, Pcg32& rng) {
 	const uint32_t scaled = (uint32_t)(pcg_next_float(rng) * (float)P.n_cascades);
-	const uint32_t level = scaled >= P.n_cascades ? scaled - P.n_cascades : scaled;
-	// the remainder by the cell count is a mask when that is a power of two (every grid the library accepts for ERP has one;
-	// an integer division costs some forty instructions, and there are up to ten here)
-	const bool pow2 = (P.n_cells & (P.n_cells - 1u)) == 0u;
-	uint32_t cell = 0, idx = 0;
-	if (pow2) grid_sample_tries<true>(i, P, n_elements, step, level, grid_in, thresh, above, tries_at_once, &cell, &idx, above_summary);
-	else grid_sample_tries<false>(i, P, n_elements, step, level, grid_in, thresh, above, tries_at_once, &cell, &idx, above_summary);
+	return scaled >= P.n_cascades ? scaled - P.n_cascades : scaled;
+}
+// the other three where it lies in the cell of the try taken
+SRF_HD Vec3 grid_sample_place(const Params& P, Pcg32& rng, uint32_t level, uint32_t cell) {
 	const uint32_t x = morton3d_invert(cell), y = morton3d_invert(cell >> 1), z = morton3d_invert(cell >> 2);
 	const float jx = pcg_next_float(rng), jy = pcg_next_float(rng), jz = pcg_next_float(rng);
 	Vec3 pos = mk3(((float)x + jx) / (float)P.grid_size[0] - 0.5f, ((float)y + jy) / (float)P.grid_size[1] - 0.5f,
@@ -252,8 +246,24 @@ SRF_HD void grid_sample_point(uint32_t i, const Params& P, uint32_t n_elements, 
 		pos = warp_position(P, pos);
 		break;
 	}
-	*position = pos;
-	*index = idx;
+	return pos;
+}
+
+// above: optional table of the comparison grid_in[idx] > thresh, one bit per cell (bit idx & 31 of word idx >> 5),
+// 32 times smaller than the grid, so that the random lookups below mostly stay in the caches
+SRF_HD void grid_sample_point(uint32_t i, const Params& P, uint32_t n_elements, Pcg32 rng, uint32_t step,
+                              const float* grid_in, float thresh, Vec3* position, uint32_t* index, const uint32_t* above = nullptr,
+                              const PcgSkip* skip = nullptr, uint32_t tries_at_once = 1,
+                             const uint64_t* skip16_m = nullptr, const uint64_t* skip16_p = nullptr, const uint32_t* above_summary = nullptr) {
+	if (skip16_m) pcg_advance_skip16(rng, i * 4u, skip16_m, skip16_p);
+	else if (skip) pcg_advance_u32(rng, i * 4u, *skip);
+	else pcg_advance(rng, (uint64_t)(uint32_t)(i * 4u));
+	const uint32_t level = grid_sample_level(P, rng);
+	const bool pow2 = (P.n_cells & (P.n_cells - 1u)) == 0u;
+	const uint32_t cell = pow2 ? grid_sample_cell<true>(i, P, n_elements, step, grid_sample_tries<true>(i, P, n_elements, step, level, grid_in, thresh, above, tries_at_once, above_summary))
+	                           : grid_sample_cell<false>(i, P, n_elements, step, grid_sample_tries<false>(i, P, n_elements, step, level, grid_in, thresh, above, tries_at_once, above_summary));
+	*position = grid_sample_place(P, rng, level, cell);
+	*index = cell + level * P.n_cells;
 }
 
 SRF_HD void grid_sample_body(uint32_t i, const Params& P, uint32_t n_elements, Pcg32 rng, uint32_t step,

@@ -65,15 +65,18 @@ __global__ void __launch_bounds__(256) k_generate_grid_samples(Params P, uint32_
 // ((i + step n) A + j B + C) mod n_cells, j = 0..9, of a random cascade: with n_cells a power of two, A odd, the points
 // whose (i + step n) A mod n_cells is v, v + 1, ... try neighbouring cells at every j, so consecutive threads read the
 // same few cache lines (one group per cascade) instead of 64 lines scattered over the grid.  Thread t = m n_cells + v
-// takes the m-th point with that v; which thread draws a point changes nothing in what is drawn.  The results go to a
-// staging array in thread order (16 bytes each, contiguous per wavefront); k_grid_samples_to_point_order then has thread i
-// fetch point i's record and write the outputs in their own order, so that neither kernel scatters its stores.
+// takes the m-th point with that v; which thread draws a point changes nothing in what is drawn.  What goes to a staging
+// array in thread order is which try was taken, one byte a point; k_grid_samples_in_point_order then has thread i fetch point i's
+// byte and work the point out, so that neither kernel scatters its stores.  Bound by the requests of that fetch, one
+// line a point where their order is not chosen for it.
+constexpr uint32_t POINT_ORDER_PER = 4;           // points a thread of k_grid_samples_in_point_order takes of a window of 1024
+constexpr uint32_t POINT_RUNS_MIN_CELLS = 1u << 22;
 constexpr uint32_t DEAL_WINDOW_MAX = 1024;      // threads of a window of k_generate_grid_samples_by_cell, at most
 // SPARSE: the launch covers a multiple of the cell count that the draw's points do not fill
 template <bool SPARSE>
 __global__ void __launch_bounds__(256) k_generate_grid_samples_by_cell(Params P, uint32_t n_elements, Pcg32 rng, uint32_t step,
                                                                         const float* __restrict__ grid_in, float thresh,
-                                                                        Float4* __restrict__ staged, const uint32_t* __restrict__ above,
+                                                                        uint8_t* __restrict__ staged, const uint32_t* __restrict__ above,
                                                                         uint32_t tries_at_once, uint32_t a_inverse, uint32_t log2_cells,
                                                                         float* __restrict__ positions, uint32_t* __restrict__ indices, uint32_t first_thread,
                                                                         uint32_t n_windows, uint32_t per) {
@@ -95,12 +98,18 @@ __global__ void __launch_bounds__(256) k_generate_grid_samples_by_cell(Params P,
 		return (uint64_t)((u - step * n_elements) & mask) + ((uint64_t)m << log2_cells);
 	};
 	auto draw = [&](uint64_t t) {
+		const uint32_t i = (uint32_t)point_of(t);
+		if (staged) {
+			Pcg32 own = rng;
+			pcg_advance_skip16(own, i * 4u, skip_m, skip_p);
+			staged[t - first_thread] = (uint8_t)grid_sample_tries<true>(i, P, n_elements, step, grid_sample_level(P, own), grid_in, thresh, above, tries_at_once);
+			return;
+		}
+		// the caller takes the points in this order (entry t of its arrays is thread t's point)
 		Vec3 pos;
 		uint32_t idx;
-		grid_sample_point((uint32_t)point_of(t), P, n_elements, rng, step, grid_in, thresh, &pos, &idx, above, nullptr, tries_at_once, skip_m, skip_p);
-		// staged == NULL: the caller takes the points in this order (entry t of its arrays is thread t's point)
-		if (staged) staged[t - first_thread] = mk4(pos.x, pos.y, pos.z, srf_u2f(idx));
-		else { st3(positions + 3 * (size_t)t, pos); indices[t] = idx; }
+		grid_sample_point(i, P, n_elements, rng, step, grid_in, thresh, &pos, &idx, above, nullptr, tries_at_once, skip_m, skip_p);
+		st3(positions + 3 * (size_t)t, pos); indices[t] = idx;
 	};
 	for (uint32_t win = blockIdx.x; win < n_windows; win += gridDim.x) {
 		const uint64_t t0 = (uint64_t)first_thread + (uint64_t)win * (per * 256u);      // staged holds the threads from first_thread on
@@ -121,17 +130,39 @@ __global__ void __launch_bounds__(256) k_generate_grid_samples_by_cell(Params P,
 	}
 }
 
-__global__ void __launch_bounds__(256) k_grid_samples_to_point_order(uint32_t n_cells, uint32_t n_elements, uint32_t step, uint32_t log2_cells,
-                                                                      const Float4* __restrict__ staged, float* __restrict__ positions, uint32_t* __restrict__ indices,
-                                                                      uint32_t first) {
+// BY_RUNS: the points' bytes lie A bytes apart (modulo the cell count), a line a point.  Runs of 32 points are therefore taken in the order
+// of where their first byte lies: run number c A^-1 (modulo the runs of a multiple) for c = 0, 1, ..., whose bytes are 32 apart from one c
+// to the next, so that a workgroup reads 32 streams of neighbouring bytes and writes whole lines.  42 M points of a 2^25-cell grid: 874 us
+// with 16 bytes staged a point, 851 us with one in the order of the points, by runs of 16, 32 and 64 311, 310 and 553 us.
+constexpr uint32_t POINT_RUN = 32;
+template <bool BY_RUNS>
+__global__ void __launch_bounds__(256) k_grid_samples_in_point_order(Params P, uint32_t n_elements, Pcg32 rng, uint32_t step, uint32_t a_inverse, uint32_t log2_cells,
+                                                                      const uint8_t* __restrict__ staged, float* __restrict__ positions, uint32_t* __restrict__ indices,
+                                                                      uint32_t first, uint32_t n_windows) {
+	__shared__ uint64_t skip_m[128], skip_p[128];
+	if (threadIdx.x < 128) pcg_skip16_entry(rng, threadIdx.x, &skip_m[threadIdx.x], &skip_p[threadIdx.x]);
+	__syncthreads();
 	// the points from `first` (a multiple of the cell count) on; staged holds the threads from `first` on
-	const uint32_t i = first + blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= n_elements) return;
-	const uint32_t mask = n_cells - 1u;
-	const uint32_t v = (((i + step * n_elements) & mask) * 56924617u) & mask;      // the inverse of the dealing above
-	const Float4 r = staged[((uint64_t)(i >> log2_cells) << log2_cells) - first + v];
-	st3(positions + 3 * (size_t)i, mk3(r.x, r.y, r.z));
-	indices[i] = srf_f2u(r.w);
+	const uint32_t mask = P.n_cells - 1u, runs = P.n_cells / POINT_RUN;
+	for (uint32_t win = blockIdx.x; win < n_windows; win += gridDim.x) {
+		#pragma unroll 2
+		for (uint32_t q = 0; q < POINT_ORDER_PER; ++q) {
+			const uint64_t t = ((uint64_t)win * POINT_ORDER_PER + q) * 256u + threadIdx.x;
+			const uint32_t run = ((uint32_t)(t / POINT_RUN) * a_inverse) & (runs - 1u);
+			const uint64_t whole = (t >> log2_cells) << log2_cells;
+			const uint64_t at = (uint64_t)first + (BY_RUNS ? whole + run * POINT_RUN + threadIdx.x % POINT_RUN : t);
+			if (at >= n_elements) continue;
+			const uint32_t i = (uint32_t)at;
+			const uint32_t v = (((i + step * n_elements) & mask) * 56924617u) & mask;      // the inverse of the dealing above
+			const uint32_t taken = staged[whole + v];
+			Pcg32 own = rng;
+			pcg_advance_skip16(own, i * 4u, skip_m, skip_p);
+			const uint32_t level = grid_sample_level(P, own);
+			const uint32_t cell = grid_sample_cell<true>(i, P, n_elements, step, taken);
+			st3(positions + 3 * (size_t)i, grid_sample_place(P, own, level, cell));
+			indices[i] = cell + level * P.n_cells;
+		}
+	}
 }
 
 // one bit per cell for each of two thresholds: bit (i & 31) of word (i >> 5) is grid[i] > thresh; 64 cells per wavefront round.
@@ -722,6 +753,7 @@ int srf_sampler_create(const srf_sampler_config* c, srf_sampler_t** out) {
 	{ const char* v = getenv("SRF_SPLAT_SORT"); if (v && v[0] == '2') s->force_splat_sort = 2; }      // 2: large-batch path through the library's sort
 	s->force_sample_bits = tri_state("SRF_GRID_SAMPLE_BITS");
 	s->force_sample_by_cell = tri_state("SRF_GRID_SAMPLE_BY_CELL");
+	{ const char* v = getenv("SRF_GRID_SAMPLE_BY_CELL"); if (v && v[0] == '2') s->force_sample_by_cell = 2; }      // 2: by cell, and back into point order by runs
 	auto team_size = [](const char* name) { const char* v = getenv(name); const uint32_t n = v && v[0] ? (uint32_t)atoi(v) : 0u; return is_pow2(n) && n <= 64u ? n : 0u; };
 	s->count_team = team_size("SRF_COUNT_TEAM");
 	s->march_team = team_size("SRF_MARCH_TEAM");
@@ -881,7 +913,7 @@ int srf_sampler_sample_positions_from_grid(srf_sampler_t* s, uint32_t n_uniform,
 	const uint64_t dealt_threads = by_cell ? (uint64_t)div_up(n_nonuniform, nc) * nc - n_dealt_b : 0;       // those that go through the staging array
 	const size_t summary_words = tabulate ? div_up(div_up(s->n_total, 32), 32) + 1 : 0;
 	const size_t summary_bytes = align_up(summary_words * 4, 256);
-	int rc = s->ws.reserve(2 * table_bytes + summary_bytes + dealt_threads * sizeof(Float4) + 256);
+	int rc = s->ws.reserve(2 * table_bytes + summary_bytes + dealt_threads + 256);
 	if (rc != SRF_OK) return rc;
 	const uint32_t* above_a = nullptr;
 	const uint32_t* above_b = nullptr;
@@ -907,7 +939,7 @@ int srf_sampler_sample_positions_from_grid(srf_sampler_t* s, uint32_t n_uniform,
 	s->dealt_entries = n_dealt;
 	if (n_dealt) {
 		hipLaunchKernelGGL(k_generate_grid_samples_by_cell<false>, dim3(dealt_grid(n_dealt / deal_window)), dim3(256), 0, st, s->P, n_uniform, s->rng, s->i_step,
-		                   (const float*)s->density_grid, -0.01f, (Float4*)nullptr, above_a, 1u, inv, log2_cells, grid_positions, grid_indices, 0u, n_dealt / deal_window, deal_window / 256u);
+		                   (const float*)s->density_grid, -0.01f, (uint8_t*)nullptr, above_a, 1u, inv, log2_cells, grid_positions, grid_indices, 0u, n_dealt / deal_window, deal_window / 256u);
 		SRF_LAUNCH_CHECK();
 	}
 	if (n_uniform > n_dealt) {
@@ -921,11 +953,11 @@ int srf_sampler_sample_positions_from_grid(srf_sampler_t* s, uint32_t n_uniform,
 	uint32_t* indices_b = grid_indices + n_uniform;
 	if (n_dealt_b) {
 		hipLaunchKernelGGL(k_generate_grid_samples_by_cell<false>, dim3(dealt_grid(n_dealt_b / deal_window)), dim3(256), 0, st, s->P, n_nonuniform, s->rng, s->i_step,
-		                   (const float*)s->density_grid, s->P.min_optical_thickness, (Float4*)nullptr, above_b, tries, inv, log2_cells, positions_b, indices_b, 0u, n_dealt_b / deal_window, deal_window / 256u);
+		                   (const float*)s->density_grid, s->P.min_optical_thickness, (uint8_t*)nullptr, above_b, tries, inv, log2_cells, positions_b, indices_b, 0u, n_dealt_b / deal_window, deal_window / 256u);
 		SRF_LAUNCH_CHECK();
 	}
 	if (by_cell) {
-		Float4* staged = (Float4*)((char*)s->ws.ptr + 2 * table_bytes + summary_bytes);
+		uint8_t* staged = (uint8_t*)s->ws.ptr + 2 * table_bytes + summary_bytes;
 		// the whole multiples of the cell count, then the one the points do not fill
 		const uint64_t full_threads = (uint64_t)n_nonuniform / nc * nc - n_dealt_b;
 		if (full_threads) {
@@ -940,8 +972,19 @@ int srf_sampler_sample_positions_from_grid(srf_sampler_t* s, uint32_t n_uniform,
 			                   (uint32_t)(n_dealt_b + full_threads), nc / deal_window, deal_window / 256u);
 			SRF_LAUNCH_CHECK();
 		}
-		hipLaunchKernelGGL(k_grid_samples_to_point_order, dim3(div_up(n_nonuniform - n_dealt_b, 256)), dim3(256), 0, st, nc, n_nonuniform, s->i_step, log2_cells,
-		                   (const Float4*)staged, positions_b, indices_b, n_dealt_b);
+		// By runs where the bytes of a multiple are more than a cache of 4 MB next to the processors holds and enough of the runs have points
+		// (us a step of drawing and updating, by runs against in order: 2^21 cells 128 / 126, a quarter of 2^25 779 / 863, of 2^26 1318 / 1544;
+		// a sixteenth of 2^25 480 / 460).  (force_sample_by_cell: either way, for the tests.)
+		bool by_runs = nc >= POINT_RUNS_MIN_CELLS && n_nonuniform - n_dealt_b >= nc / 8u;
+		if (s->force_sample_by_cell > 0) by_runs = s->force_sample_by_cell == 2;
+		const uint64_t threads = by_runs ? dealt_threads : n_nonuniform - n_dealt_b;
+		const uint32_t windows = (uint32_t)((threads + 256u * POINT_ORDER_PER - 1u) / (256u * POINT_ORDER_PER)), groups = windows < 16384u ? windows : 16384u;
+		if (by_runs)
+			hipLaunchKernelGGL(k_grid_samples_in_point_order<true>, dim3(groups), dim3(256), 0, st, s->P, n_nonuniform, s->rng, s->i_step, inv, log2_cells, (const uint8_t*)staged,
+			                   positions_b, indices_b, n_dealt_b, windows);
+		else
+			hipLaunchKernelGGL(k_grid_samples_in_point_order<false>, dim3(groups), dim3(256), 0, st, s->P, n_nonuniform, s->rng, s->i_step, inv, log2_cells, (const uint8_t*)staged,
+			                   positions_b, indices_b, n_dealt_b, windows);
 		SRF_LAUNCH_CHECK();
 	} else if (n_nonuniform > n_dealt_b) {
 		const uint32_t runs = div_up(n_nonuniform - n_dealt_b, 256);

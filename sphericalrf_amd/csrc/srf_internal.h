@@ -55,7 +55,8 @@ struct srf_sampler {
 	bool     skip_enabled;  // SRF_MARCH_SKIP=0 in the environment at creation switches the table off
 	// Switches the tests use to run both sides of a size-dependent choice on small inputs; read from the environment once, when the
 	// sampler is created (-1: the library chooses): SRF_SPLAT_SORT, SRF_GRID_SAMPLE_BITS, SRF_GRID_SAMPLE_BY_CELL = 0|1
-	// (SRF_SPLAT_SORT=2: the large-batch splat through the library's radix sort instead of the partition made for it);
+	// (SRF_SPLAT_SORT=2: the large-batch splat through the library's radix sort instead of the partition made for it;
+	// SRF_GRID_SAMPLE_BY_CELL=2: points dealt by cell brought back into their order by runs, as on large grids);
 	// SRF_COUNT_TEAM, SRF_MARCH_TEAM = lanes a ray of the counting march, of the render marches begins with (a power of two up to 64)
 	int      force_splat_sort, force_sample_bits, force_sample_by_cell;
 	uint32_t count_team = 0;
